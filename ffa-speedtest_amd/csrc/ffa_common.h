@@ -69,50 +69,22 @@ __device__ __forceinline__ float round_to(float v, int dt) {
 }
 
 // ---------------------------------------------------------------------------
-// fp8 (OCP e4m3fn / e5m2) encode with torch's rules: RNE, e4m3fn overflow -> NaN,
-// e5m2 overflow -> inf.  Written from the format definitions.
+// fp8 (OCP e4m3fn / e5m2) encode with torch's rules: RNE, e4m3fn overflow -> NaN, e5m2 overflow ->
+// inf, a NaN's byte its sign and 0x7f.  gfx950 converts a pair with one v_cvt_pk_fp8_f32 /
+// v_cvt_pk_bf8_f32; over all 2^32 fp32 patterns its bytes are these for everything but NaN inputs
+// (always 0xff / 0xfe), which are put right.  A conversion in integer arithmetic from the format
+// definitions is some 25 instructions an element with two branches: with it the nvfp4 quantizer of
+// 20K x 1024 bf16 keys took 124.6 us a call, with this 103.8 (the 2-bit one of 32K x 1024: 337 -> 311).
 // ---------------------------------------------------------------------------
+template <bool E4M3>
+__device__ __forceinline__ uint32_t fp8_pair_hw(float a, float b) {  // bytes of a (low) and b; NaN signs not kept
+  if constexpr (E4M3) return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false) & 0xffffu;
+  else return (uint32_t)__builtin_amdgcn_cvt_pk_bf8_f32(a, b, 0, false) & 0xffffu;
+}
 __device__ __forceinline__ uint32_t f32_to_fp8(float x, int e4m3) {
   const uint32_t u = __float_as_uint(x);
-  const uint32_t sign = (u >> 24) & 0x80u;
-  const uint32_t a = u & 0x7fffffffu;
-  const int mbits = e4m3 ? 3 : 2;
-  const int bias = e4m3 ? 7 : 15;
-  const int emin = 1 - bias;  // smallest normal exponent
-  if (a > 0x7f800000u) return sign | 0x7fu;  // NaN
-  if (a == 0x7f800000u) return e4m3 ? (sign | 0x7fu) : (sign | 0x7cu);
-  const int e = (int)(a >> 23) - 127;  // unbiased exponent of the input (normal inputs)
-  uint32_t bits;
-  if (a < 0x00800000u || e < emin) {
-    // result is subnormal (or zero) in fp8: a multiple of the quantum 2^(emin - mbits),
-    // rounded to nearest even in units of the quantum
-    const float q = __uint_as_float((uint32_t)(127 + emin - mbits) << 23);  // 2^(emin-mbits)
-    const float r = __uint_as_float(a) / q;                                 // exact (power of 2)
-    const float ri = __builtin_rintf(r);                                    // RNE
-    bits = (uint32_t)ri;  // may equal 1 << mbits => smallest normal, encodes correctly
-  } else {
-    // normal: keep mbits of mantissa with RNE
-    const uint32_t shift = 23 - mbits;
-    uint32_t mant = a & 0x7fffffu;
-    uint32_t keep = mant >> shift;
-    const uint32_t rem = mant & ((1u << shift) - 1u);
-    const uint32_t half = 1u << (shift - 1);
-    uint32_t exp8 = (uint32_t)(e + bias);
-    if (rem > half || (rem == half && (keep & 1u))) {
-      keep += 1;
-      if (keep == (1u << mbits)) {
-        keep = 0;
-        exp8 += 1;
-      }
-    }
-    bits = (exp8 << mbits) | keep;
-  }
-  if (e4m3) {
-    if (bits > 0x7eu) return sign | 0x7fu;  // beyond 448 -> NaN
-  } else {
-    if (bits > 0x7bu) return sign | 0x7cu;  // beyond 57344 -> inf
-  }
-  return sign | bits;
+  const uint32_t b = (e4m3 ? fp8_pair_hw<true>(x, x) : fp8_pair_hw<false>(x, x)) & 0xffu;
+  return (u & 0x7fffffffu) > 0x7f800000u ? ((u >> 24) & 0x80u) | 0x7fu : b;
 }
 
 // ---------------------------------------------------------------------------
