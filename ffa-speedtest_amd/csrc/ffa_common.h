@@ -87,6 +87,80 @@ __device__ __forceinline__ uint32_t f32_to_fp8(float x, int e4m3) {
   return (u & 0x7fffffffu) > 0x7f800000u ? ((u >> 24) & 0x80u) | 0x7fu : b;
 }
 
+// Eight floats to eight fp8 bytes in memory order.  A NaN among them (seen in the sum, which other
+// than for NaNs is only a NaN for infinities of both signs) takes the element-wise conversion, which
+// keeps its sign.
+template <bool E4M3>
+__device__ __forceinline__ uint2 f32x8_to_fp8(const float *x) {
+  uint2 w;
+  if constexpr (E4M3) {
+    w.x = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(x[2], x[3], __builtin_amdgcn_cvt_pk_fp8_f32(x[0], x[1], 0, false), true);
+    w.y = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(x[6], x[7], __builtin_amdgcn_cvt_pk_fp8_f32(x[4], x[5], 0, false), true);
+  } else {
+    w.x = (uint32_t)__builtin_amdgcn_cvt_pk_bf8_f32(x[2], x[3], __builtin_amdgcn_cvt_pk_bf8_f32(x[0], x[1], 0, false), true);
+    w.y = (uint32_t)__builtin_amdgcn_cvt_pk_bf8_f32(x[6], x[7], __builtin_amdgcn_cvt_pk_bf8_f32(x[4], x[5], 0, false), true);
+  }
+  const float any = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+  if (__builtin_isnan(any)) [[unlikely]] {
+    w = make_uint2(0u, 0u);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      w.x |= f32_to_fp8(x[e], E4M3) << (8 * e);
+      w.y |= f32_to_fp8(x[4 + e], E4M3) << (8 * e);
+    }
+  }
+  return w;
+}
+
+// Eight consecutive elements of a float tensor of dtype DT (0=f16, 1=bf16, 2=f32) at an address that is
+// a multiple of their size: one or two 16-byte loads, then conversions that need no dtype test.
+template <int DT>
+struct Raw8 {
+  uint4 v[DT == 2 ? 2 : 1];
+};
+template <int DT>
+__device__ __forceinline__ Raw8<DT> load8(const void *p, size_t i) {
+  Raw8<DT> r;
+  const uint4 *s = (const uint4 *)((const uint8_t *)p + i * (DT == 2 ? 4 : 2));
+  r.v[0] = s[0];
+  if constexpr (DT == 2) r.v[1] = s[1];
+  return r;
+}
+template <int DT>
+__device__ __forceinline__ void raw8_to_f32(const Raw8<DT> &r, float *x) {
+  if constexpr (DT == 2) {
+    const uint32_t w[8] = {r.v[0].x, r.v[0].y, r.v[0].z, r.v[0].w, r.v[1].x, r.v[1].y, r.v[1].z, r.v[1].w};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = __uint_as_float(w[e]);
+  } else {
+    const uint32_t w[4] = {r.v[0].x, r.v[0].y, r.v[0].z, r.v[0].w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x[2 * e] = DT == 1 ? __uint_as_float(w[e] << 16) : f16_bits_to_f32(w[e] & 0xffffu);
+      x[2 * e + 1] = DT == 1 ? __uint_as_float(w[e] & 0xffff0000u) : f16_bits_to_f32(w[e] >> 16);
+    }
+  }
+}
+// eight floats rounded to dtype DT and back (the hardware's paired conversions: RNE)
+template <int DT>
+__device__ __forceinline__ void round8(float *x) {
+  if constexpr (DT != 2) {
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {
+      if constexpr (DT == 1) {
+        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+        const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x[e], x[e + 1]}, bf16x2));
+        x[e] = __uint_as_float(w << 16);
+        x[e + 1] = __uint_as_float(w & 0xffff0000u);
+      } else {
+        const uint32_t w = pk_f16_bits(x[e], x[e + 1]);
+        x[e] = f16_bits_to_f32(w & 0xffffu);
+        x[e + 1] = f16_bits_to_f32(w >> 16);
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // lane exchange
 // ---------------------------------------------------------------------------

@@ -44,16 +44,28 @@ __global__ __launch_bounds__(256) void q2_minmax_kernel(const void *k, int kdt, 
   minmax[((size_t)(B + b) * nsplit + split) * C + c] = mx;
 }
 
+// 32 columns per workgroup, 8 threads a column: the splits' extrema are read 8 at a time instead of one
+// after the other (64 splits of 1024 columns: 17.5 us as a chain of dependent reads by 4 workgroups)
 __global__ __launch_bounds__(256) void q2_scale_kernel(const float *minmax, int B, int nsplit, int C, int kdt,
                                                         void *scale, void *zero) {
   const int b = blockIdx.y;
-  const int c = blockIdx.x * 256 + threadIdx.x;
-  if (c >= C) return;
+  const int col = threadIdx.x & 31, r = threadIdx.x >> 5;
+  const int c = blockIdx.x * 32 + col;
   float mn = INFINITY, mx = -INFINITY;
-  for (int s = 0; s < nsplit; ++s) {
-    mn = fminf(mn, minmax[((size_t)b * nsplit + s) * C + c]);
-    mx = fmaxf(mx, minmax[((size_t)(B + b) * nsplit + s) * C + c]);
+  if (c < C) {
+#pragma unroll 8
+    for (int s = r; s < nsplit; s += 8) {
+      mn = fminf(mn, minmax[((size_t)b * nsplit + s) * C + c]);
+      mx = fmaxf(mx, minmax[((size_t)(B + b) * nsplit + s) * C + c]);
+    }
   }
+  __shared__ float s_m[2][8][32];
+  s_m[0][r][col] = mn;
+  s_m[1][r][col] = mx;
+  __syncthreads();
+  if (r != 0 || c >= C) return;
+#pragma unroll
+  for (int i = 1; i < 8; ++i) mn = fminf(mn, s_m[0][i][col]), mx = fmaxf(mx, s_m[1][i][col]);
   // scale = tau(tau(tau(max - min).clamp_min(1e-6)) / 3.0)   (run_attn_bench_q2.py:82)
   const float diff = round_to(mx - mn, kdt);
   const float cl = round_to(fmaxf(diff, 1e-6f), kdt);
@@ -99,6 +111,116 @@ __global__ __launch_bounds__(256) void q2_quant_channel_kernel(const void *k, in
   const int b = (int)(row / ((size_t)HKV * T));
   quant_channel_byte(k, kdt, row, D, byte, scale, zero, ((size_t)b * HKV + hkv) * D, kq + row * DP + byte,
                      res + row * D, res_e4m3);
+}
+
+// ---- the same quantizer over vectors of 8 columns (D a multiple of 4, HKV * D a multiple of 8, aligned
+// pointers): columns of a [B, T, C = HKV * D] tensor are quantized independently, so the kernels see C
+// only.  Both passes are bound by reading K and writing codes and residual once; what kept the scalar
+// kernels from it were 2-byte loads one after the other (minimum / maximum of 32K x 1024 bf16: 150 us)
+// and, per element, an IEEE division and two roundings in software (112 us).
+
+// Minimum and maximum per column of one split of the tokens: a workgroup covers 128 columns (256 or 512
+// bytes of a row, 16 lanes), 16 token rows at a time, 8 of them in flight per lane.
+constexpr int kMmCols = 128, kMmRows = 16, kMmFly = 8;
+template <int KDT>
+__global__ __launch_bounds__(256) void q2_minmax8_kernel(const void *k, int T, int C, int nsplit, float *minmax) {
+  const int split = blockIdx.x, b = blockIdx.y, B = gridDim.y;
+  const int cl = (threadIdx.x & 15) * 8, c = blockIdx.z * kMmCols + cl, r = threadIdx.x >> 4;
+  const int tper = (T + nsplit - 1) / nsplit;
+  const int ta = split * tper, tb = min(T, ta + tper);
+  float mn[8], mx[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) mn[e] = INFINITY, mx[e] = -INFINITY;
+  if (c < C) {
+    for (int t = ta + r; t < tb; t += kMmRows * kMmFly) {
+      Raw8<KDT> w[kMmFly];
+#pragma unroll
+      for (int u = 0; u < kMmFly; ++u)  // rows past the split repeat its last: no effect on an extremum
+        w[u] = load8<KDT>(k, ((size_t)b * T + min(t + kMmRows * u, tb - 1)) * C + c);
+#pragma unroll
+      for (int u = 0; u < kMmFly; ++u) {
+        float x[8];
+        raw8_to_f32<KDT>(w[u], x);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) mn[e] = fminf(mn[e], x[e]), mx[e] = fmaxf(mx[e], x[e]);
+      }
+    }
+  }
+  __shared__ float s_mn[kMmRows][kMmCols + 4], s_mx[kMmRows][kMmCols + 4];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) s_mn[r][cl + e] = mn[e], s_mx[r][cl + e] = mx[e];
+  __syncthreads();
+  const int col = threadIdx.x & (kMmCols - 1), cc = blockIdx.z * kMmCols + col;
+  const bool lo = threadIdx.x < kMmCols;
+  float m = lo ? s_mn[0][col] : s_mx[0][col];
+#pragma unroll
+  for (int i = 1; i < kMmRows; ++i) m = lo ? fminf(m, s_mn[i][col]) : fmaxf(m, s_mx[i][col]);
+  if (cc < C) minmax[((size_t)(lo ? b : B + b) * nsplit + split) * C + cc] = m;
+}
+
+// Smallest float x with code(x) >= i + 1 for a scale sc > 0, where code(x) = clamp(rne(tau(x / sc)), 0, 3),
+// the quotient in fp32 first (one division per element in the reference, run_attn_bench_q2.py:84-85).
+// The code is monotone in x, and it turns where tau(x / sc) passes 0.5, 1.5, 2.5 (ties to even: above 0.5,
+// at 1.5, above 2.5), i.e. where x / sc passes the middle of the tau values around: q = 0.5 + u/2 (above),
+// 1.5 - u'/2 (at or above), 2.5 + u''/2 (above), with the ulps u of tau there.  q * sc is exact in
+// double, and for fp16 / bf16 the fp32 quotient does not cross q (x and sc have at most 11 bits, so x / sc
+// is q or at least 2^-24 away from it).  A scale that is not finite gives a NaN, which no x passes, as
+// x / inf = 0 and inf / inf = NaN take code 0.
+template <int KDT>
+__device__ __forceinline__ float q2_turn(float sc, int i) {
+  constexpr int p = KDT == 2 ? 24 : (KDT == 1 ? 8 : 11);  // significant bits of tau
+  constexpr double h = 1.0 / (double)(1u << p);           // an ulp of tau in [1/2, 1)
+  const double q = i == 0 ? 0.5 + 0.5 * h : (i == 1 ? 1.5 - h : 2.5 + 2.0 * h);
+  const double v = (double)sc * q;
+  float f = (float)v;
+  const bool up = i == 1 ? (double)f < v : (double)f <= v;
+  if (up) f = __uint_as_float(__float_as_uint(f) + 1u);
+  return sc < INFINITY ? f : __builtin_nanf("");
+}
+
+// Codes and residual: a lane keeps the scale, zero point and the three turning points of its 8 columns and
+// walks down the tokens, so an element costs a subtraction, a rounding, three compares and half an fp8
+// conversion.  A wave reads 64 consecutive vectors (1 or 2 KB) and writes 512 residual and 128 code bytes.
+template <int KDT, bool E4M3>
+__global__ __launch_bounds__(256) void q2_quant8_kernel(const void *k, int T, int C, int lw, int per, const void *scale,
+                                                        const void *zero, uint8_t *kq, uint8_t *res) {
+  const int b = blockIdx.z;
+  const int chunk = (blockIdx.y << lw) + (threadIdx.x & ((1 << lw) - 1));
+  const int rows = 256 >> lw, c = chunk * 8;
+  if (c >= C) return;
+  float sc[8], zr[8], turn[3][8];
+  raw8_to_f32<KDT>(load8<KDT>(scale, (size_t)b * C + c), sc);
+  raw8_to_f32<KDT>(load8<KDT>(zero, (size_t)b * C + c), zr);
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) turn[i][e] = q2_turn<KDT>(sc[e], i);
+  const int ta = blockIdx.x * per, tb = min(T, ta + per);
+  constexpr int kFly = KDT == 2 ? 2 : 4;  // token rows in flight per lane
+  for (int t = ta + (threadIdx.x >> lw); t < tb; t += rows * kFly) {
+    Raw8<KDT> w[kFly];
+#pragma unroll
+    for (int u = 0; u < kFly; ++u) w[u] = load8<KDT>(k, ((size_t)b * T + min(t + rows * u, tb - 1)) * C + c);
+#pragma unroll
+    for (int u = 0; u < kFly; ++u) {
+      if (t + rows * u >= tb) break;
+      float kv[8], xs[8], d[8];
+      raw8_to_f32<KDT>(w[u], kv);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) xs[e] = kv[e] - zr[e];  // (k - zero) in tau
+      round8<KDT>(xs);
+      uint32_t packed = 0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t cq = xs[e] >= turn[2][e] ? 3u : (xs[e] >= turn[1][e] ? 2u : (xs[e] >= turn[0][e] ? 1u : 0u));
+        d[e] = kv[e] - ((float)cq * sc[e] + zr[e]);  // two fp32 roundings of the dequantized value
+        packed |= cq << (2 * e);
+      }
+      const size_t row = (size_t)b * T + t + rows * u;
+      *(uint2 *)(res + row * C + c) = f32x8_to_fp8<E4M3>(d);
+      *(uint16_t *)(kq + row * (C >> 2) + 2 * chunk) = (uint16_t)packed;
+    }
+  }
 }
 
 // Reference-layout append: token n of sequence b (k_new [B, Tn, HKV, D]) is quantized with the
@@ -437,18 +559,58 @@ extern "C" int ffa_q2_quantize_nsplit(int T) {
   return s < 1 ? 1 : (s > 64 ? 64 : s);
 }
 
+// the vector kernels of one K dtype
+template <int KDT>
+static void launch_quant8(const void *k, int B, int T, int C, int nsplit, uint8_t *k_q, void *scale, void *zero,
+                          uint8_t *residual, bool e4m3, float *minmax, hipStream_t st) {
+  hipLaunchKernelGGL(ffa::q2_minmax8_kernel<KDT>, dim3(nsplit, B, (C + ffa::kMmCols - 1) / ffa::kMmCols), dim3(256), 0,
+                     st, k, T, C, nsplit, minmax);
+  hipLaunchKernelGGL(ffa::q2_scale_kernel, dim3((C + 31) / 32, B), dim3(256), 0, st, (const float *)minmax, B, nsplit,
+                     C, KDT, scale, zero);
+  // a workgroup covers 2^lw vectors of a row and 256 >> lw rows at a time; its tokens: enough that a lane's
+  // turning points are paid over 16 rows, but no fewer than 1024 workgroups while rows remain
+  const int c8 = C / 8;
+  int lw = 0;
+  while (lw < 6 && (1 << lw) < c8) ++lw;
+  const int rows = 256 >> lw, ny = (c8 + (1 << lw) - 1) >> lw;
+  const long units = (long)B * ny * ((T + rows - 1) / rows);  // row steps of all workgroups
+  long steps = units / 1024;
+  steps = steps < 1 ? 1 : (steps > 16 ? 16 : steps);
+  const int per = (int)steps * rows;
+  const dim3 grid((unsigned)((T + per - 1) / per), (unsigned)ny, (unsigned)B);
+  if (e4m3)
+    hipLaunchKernelGGL((ffa::q2_quant8_kernel<KDT, true>), grid, dim3(256), 0, st, k, T, C, lw, per,
+                       (const void *)scale, (const void *)zero, k_q, residual);
+  else
+    hipLaunchKernelGGL((ffa::q2_quant8_kernel<KDT, false>), grid, dim3(256), 0, st, k, T, C, lw, per,
+                       (const void *)scale, (const void *)zero, k_q, residual);
+}
+
+static bool aligned(const void *p, size_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
+
 static int launch_quant_channel(const void *k, int kdt, int B, int T, int HKV, int D, uint8_t *k_q, void *scale,
                                 void *zero, uint8_t *residual, int res_dtype, float *minmax, hipStream_t st) {
   const int C = HKV * D;
   const int nsplit = ffa_q2_quantize_nsplit(T);
-  hipLaunchKernelGGL(ffa::q2_minmax_kernel, dim3(nsplit, B, (C + 255) / 256), dim3(256), 0, st, k, kdt, T, C, nsplit,
-                     minmax);
-  hipLaunchKernelGGL(ffa::q2_scale_kernel, dim3((C + 255) / 256, B), dim3(256), 0, st, (const float *)minmax, B,
-                     nsplit, C, kdt, scale, zero);
-  const size_t total = (size_t)B * T * HKV * ((D + 3) / 4);
-  hipLaunchKernelGGL(ffa::q2_quant_channel_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, k, kdt, B,
-                     T, HKV, D, (const void *)scale, (const void *)zero, k_q, residual,
-                     res_dtype == FFA_DT_FP8_E4M3 ? 1 : 0);
+  const int e4m3 = res_dtype == FFA_DT_FP8_E4M3 ? 1 : 0;
+  // vectors of 8 columns: whole code bytes (D), whole vectors (C), aligned loads and stores, grid limits
+  if (D % 4 == 0 && C % 8 == 0 && B <= 65535 && C <= 65535 * ffa::kMmCols && aligned(k, 16) && aligned(scale, 16) &&
+      aligned(zero, 16) && aligned(residual, 8) && aligned(k_q, 2)) {
+    if (kdt == FFA_DT_F16)
+      launch_quant8<FFA_DT_F16>(k, B, T, C, nsplit, k_q, scale, zero, residual, e4m3 != 0, minmax, st);
+    else if (kdt == FFA_DT_BF16)
+      launch_quant8<FFA_DT_BF16>(k, B, T, C, nsplit, k_q, scale, zero, residual, e4m3 != 0, minmax, st);
+    else
+      launch_quant8<FFA_DT_F32>(k, B, T, C, nsplit, k_q, scale, zero, residual, e4m3 != 0, minmax, st);
+  } else {
+    hipLaunchKernelGGL(ffa::q2_minmax_kernel, dim3(nsplit, B, (C + 255) / 256), dim3(256), 0, st, k, kdt, T, C, nsplit,
+                       minmax);
+    hipLaunchKernelGGL(ffa::q2_scale_kernel, dim3((C + 31) / 32, B), dim3(256), 0, st, (const float *)minmax, B,
+                       nsplit, C, kdt, scale, zero);
+    const size_t total = (size_t)B * T * HKV * ((D + 3) / 4);
+    hipLaunchKernelGGL(ffa::q2_quant_channel_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, k, kdt,
+                       B, T, HKV, D, (const void *)scale, (const void *)zero, k_q, residual, e4m3);
+  }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return ffa_set_error_internal(FFA_E_LAUNCH, hipGetErrorString(e));
   return FFA_OK;

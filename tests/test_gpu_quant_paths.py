@@ -7,8 +7,6 @@ import torch
 from helpers import FP8_DT, TORCH_DT, f32
 from oracle import formats as OF
 
-pytestmark = pytest.mark.gpu
-
 
 def _u8(t):
     return t.contiguous().view(torch.uint8).cpu().numpy()
@@ -23,6 +21,7 @@ def _edge_floats():
     return np.concatenate(parts).view(np.float32)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("fmt", ["e4m3fn", "e5m2"])
 def test_fp8_bytes_of_edge_values(gpu, fmt):
     """base = fp8(k) byte for byte, NaN signs included (the residual of a NaN or an overflow is a NaN whose
@@ -36,3 +35,89 @@ def test_fp8_bytes_of_edge_values(gpu, fmt):
     assert np.array_equal(_u8(base), ob)
     fine = (ob & 0x7F) < (0x7F if fmt == "e4m3fn" else 0x7C)
     assert np.array_equal(_u8(res)[fine], orr[fine])
+
+
+# ------------------------------------------------------------------- per-channel 2-bit quantizer
+def _misaligned(k):
+    """The same values at an address that is no multiple of 16 bytes (the scalar kernels' route)."""
+    flat = torch.empty(k.numel() + 1, dtype=k.dtype, device=k.device)
+    flat[1:] = k.reshape(-1)
+    return flat[1:].view(k.shape)
+
+
+def _next(x, tau, n):
+    """x moved by n representable values of tau (x positive)."""
+    if tau == "fp32":
+        return (x.view(torch.int32) + n).view(torch.float32)
+    return (x.view(torch.int16) + n).view(x.dtype)
+
+
+def test_q2_code_turning_points():
+    """The closed form the vector quantizer compares against (the middles of the tau values around 0.5, 1.5 and
+    2.5, times the scale) gives, for every 16-bit scale and a sample of fp32 ones, the code that the division gives
+    on both sides of every turn."""
+    g = torch.Generator().manual_seed(5)
+    for tau in ("bf16", "fp16", "fp32"):
+        dt, p = TORCH_DT[tau], {"bf16": 8, "fp16": 11, "fp32": 24}[tau]
+        if tau == "fp32":
+            sc = torch.rand(20000, generator=g) * torch.exp2(torch.randint(-20, 20, (20000,), generator=g).float())
+            sc = torch.cat([sc.clamp_min(3e-7), torch.exp2(torch.arange(-20, 20).float())])
+        else:
+            sc = torch.arange(1, 0x7C00 if tau == "fp16" else 0x7F00, dtype=torch.int16).view(dt)
+            sc = sc[(sc.float() >= 3e-7) & (sc.float() < 1e4)]
+        h = 2.0 ** -p
+        for i, q in enumerate((0.5 + h / 2, 1.5 - h, 2.5 + 2 * h)):
+            v = sc.double() * q
+            t = v.float()
+            up = t.double() < v if i == 1 else t.double() <= v
+            t = torch.where(up, (t.view(torch.int32) + 1).view(torch.float32), t)
+            near = (sc.float() * (i + 0.5)).to(dt)
+            for n in range(-3, 4):
+                x = _next(near, tau, n)
+                code = torch.round(x / sc).clamp(0, 3)  # the reference's ops in tau
+                assert torch.equal(x.float() >= t, code.float() >= i + 1), (tau, i, n)
+
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tau", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("fmt", ["e4m3fn", "e5m2"])
+def test_q2_quantizer_turning_points_bit_exact(gpu, tau, fmt):
+    """Keys on and next to every code's turning point of 4096 scales, against the oracle."""
+    from ffa_mi355x.quant import quantize_per_channel
+    from oracle import q2fp8 as OQ
+
+    dt = TORCH_DT[tau]
+    g = torch.Generator().manual_seed(11)
+    sc = (torch.rand(4, 8, 128, generator=g) * 4 + 0.01).to(dt)
+    rows = [torch.zeros_like(sc), (sc.float() * 3).to(dt)]  # zero 0, scale tau(tau(3 sc) / 3)
+    s1 = (rows[1] / 3.0)
+    for mid in (0.5, 1.5, 2.5):
+        rows += [_next((s1.float() * mid).to(dt), tau, n) for n in range(-3, 4)]
+    k = torch.stack(rows, 1)  # [4, T, 8, 128]
+    kq, ks, kz, kr = quantize_per_channel(k.to(gpu), FP8_DT[fmt])
+    oq, os_, oz, orr = OQ.quantize_per_channel(f32(k), tau, fmt)
+    assert np.array_equal(_u8(kq), oq) and np.array_equal(_u8(kr), orr)
+    assert np.array_equal(f32(ks), os_) and np.array_equal(f32(kz), oz)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tau", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("B,T,HKV,D", [(1, 1, 1, 8), (2, 257, 3, 24), (1, 300, 2, 12), (3, 17, 5, 64), (1, 2500, 8, 128),
+                                       (2, 129, 9, 128)])
+def test_q2_quantizer_vector_route_equals_scalar_route(gpu, tau, B, T, HKV, D):
+    """Every byte of the vector kernels' route equals the scalar route's, tails of columns, rows and splits,
+    infinities and NaNs among them."""
+    from ffa_mi355x.quant import quantize_per_channel
+
+    g = torch.Generator().manual_seed(B * 1000 + T)
+    k = (torch.randn(B, T, HKV, D, generator=g) * 3).to(TORCH_DT[tau])
+    if T > 16:
+        k[0, 3, 0, 1], k[0, 5, 0, 2], k[-1, 7, HKV - 1, 3], k[0, 9, 0, 4] = float("inf"), float("-inf"), float("nan"), 0.0
+        k[0, 11, 0, 5:7] = 6e4
+        k[0, 12, 0, 6] = -6e4
+    k = k.to(gpu)
+    for fp8 in (torch.float8_e5m2, torch.float8_e4m3fn):
+        a, b = quantize_per_channel(k, fp8), quantize_per_channel(_misaligned(k), fp8)
+        for x, y in zip(a, b):
+            assert np.array_equal(_u8(x), _u8(y))
