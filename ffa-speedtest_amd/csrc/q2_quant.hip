@@ -117,7 +117,8 @@ __global__ __launch_bounds__(256) void q2_quant_channel_kernel(const void *k, in
 // pointers): columns of a [B, T, C = HKV * D] tensor are quantized independently, so the kernels see C
 // only.  Both passes are bound by reading K and writing codes and residual once; what kept the scalar
 // kernels from it were 2-byte loads one after the other (minimum / maximum of 32K x 1024 bf16: 150 us)
-// and, per element, an IEEE division and two roundings in software (112 us).
+// and, per element, an IEEE division and two roundings in software (112 us).  A call on 32K x 1024 bf16 keys
+// (109 MB read and written once) took 341 us with the scalar kernels and takes 38 with these.
 
 // Minimum and maximum per column of one split of the tokens: a workgroup covers 128 columns (256 or 512
 // bytes of a row, 16 lanes), 16 token rows at a time, 8 of them in flight per lane.
@@ -417,6 +418,199 @@ __global__ __launch_bounds__(512) void kproj_rope_kernel(const void *h, const vo
   }
 }
 
+// The same for many tokens: a tile of TM tokens x TN output channels per 256-thread workgroup, operands
+// staged through LDS.  (The kernel above keeps few tokens' W stream spread over the chip; with many it
+// reads h and W from the caches once per 32 channels and 16 tokens: 4096 tokens x 4096 -> 1024 take 249 us
+// there and 53 here, 0.65 PFLOP/s; the matrix cores need 23 at the rate a large product reaches.  What is
+// left: of a 64-wide step's 1320 cycles 512 are products, LDS moves 96 KB in another 515, partly under
+// them, and a wave has its SIMD to itself, so that every wait shows; 8 us are the first loads and the end.)
+//   * Four waves in 2 x 2 quarters; MFMA rows are channels and columns are tokens, so that a lane ends with
+//     four consecutive channels of one token: RoPE pairs need no exchange, stores are 16 bytes (fp32).
+//   * K in steps of 64: 16-byte pieces go to registers four steps ahead and to one of three LDS buffers two
+//     steps ahead, one barrier a step; a step's operands are read under the products before them (with two
+//     buffers, and the reads and writes between the products, 57 us).  A row's eight pieces are stored at
+//     piece ^ (row & 7), so that the 16 rows an operand read touches spread over the banks (no conflicts).
+//   * Accumulators are folded into a second set every kGemmFold steps: chains as long as the split over
+//     eight waves gives at H = 4096, and its rounding error.
+//   * Workgroups go round-robin to the 8 XCDs; each XCD takes a run of consecutive tiles, channel tiles
+//     fastest, so that its L2 serves a tile row's tokens to every channel tile.
+constexpr int kGemmK = 64, kGemmFold = 8;
+
+template <int HDT, bool CS32, int TM, int TN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void kproj_rope_tile_kernel(
+    const void *h, const void *w, const void *bias, const void *cos, const void *sin, int M, int T, int H, int N, int D,
+    void *kout) {
+  constexpr int kRow = kGemmK * 2;                    // bytes of a staged row
+  constexpr int kPa = TN * 8 / 256, kPb = TM * 8 / 256;  // 16-byte pieces per thread and step: W, h
+  constexpr int kMi = TN / 32, kNi = TM / 32;         // MFMA tiles of a wave: channels, tokens
+  constexpr int kBuf = (TM + TN) * kRow;
+  __shared__ __attribute__((aligned(16))) uint8_t s_t[3 * kBuf];
+  const int nct = (N + TN - 1) / TN;
+  int tile = blockIdx.x;
+  if ((gridDim.x & 7) == 0) tile = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
+  const int n0 = (tile % nct) * TN, m0 = (tile / nct) * TM;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int wn = (wv & 1) * (TN / 2), wm = (wv >> 1) * (TM / 2);
+
+  // pieces of this thread: piece i of an operand is row (threadIdx.x + 256 i) / 8, 16-byte column % 8; rows
+  // past the end read zeros (never stored)
+  const int pr = threadIdx.x >> 3, pc = threadIdx.x & 7;
+  const brsrc rw = make_rsrc((const uint16_t *)w + (size_t)n0 * H, (uint32_t)(min(TN, N - n0) * H * 2));
+  const brsrc rh = make_rsrc((const uint16_t *)h + (size_t)m0 * H, (uint32_t)(min(TM, M - m0) * H * 2));
+  const uint32_t src = (uint32_t)(pr * H * 2 + pc * 16), src32 = (uint32_t)(64 * H);  // bytes of 32 rows
+  const uint32_t dst = (uint32_t)(pr * kRow + ((pc ^ (pr & 7)) * 16));  // + 32 rows per piece (32 is a multiple of 8)
+  u32x4 a0[kPa], b0[kPb], a1[kPa], b1[kPb];  // steps of even and odd number
+  const int steps = H / kGemmK;
+  auto fetch = [&](u32x4(&a)[kPa], u32x4(&b)[kPb], int step) {
+    const int k = min(step, steps - 1) * kRow;
+#pragma unroll
+    for (int i = 0; i < kPa; ++i) a[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(src + src32 * i), k, 0);
+#pragma unroll
+    for (int i = 0; i < kPb; ++i) b[i] = __builtin_amdgcn_raw_buffer_load_b128(rh, (int)(src + src32 * i), k, 0);
+  };
+  auto stage = [&](const u32x4(&a)[kPa], const u32x4(&b)[kPb], uint8_t *to) {
+#pragma unroll
+    for (int i = 0; i < kPa; ++i) *(u32x4 *)(to + dst + 32 * kRow * i) = a[i];
+#pragma unroll
+    for (int i = 0; i < kPb; ++i) *(u32x4 *)(to + TN * kRow + dst + 32 * kRow * i) = b[i];
+  };
+  // LDS traffic only (lgkmcnt 0, the loads of later steps stay in flight), and with the builtin wait, so
+  // that the compiler counts on from it
+  auto lds_barrier = []() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  f32x4 acc[kMi][kNi], sum[kMi][kNi];
+#pragma unroll
+  for (int i = 0; i < kMi; ++i)
+#pragma unroll
+    for (int j = 0; j < kNi; ++j) acc[i][j] = sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int fr = lane & 15, fq = lane >> 4;
+  const uint32_t fo[2] = {(uint32_t)((fq ^ (fr & 7)) * 16), (uint32_t)(((4 + fq) ^ (fr & 7)) * 16)};
+  uint4 fa[2][kMi], fb[2][kNi];  // operands of the two 32-wide halves of a step
+  auto read = [&](int kk, const uint8_t *from) {
+    const uint8_t *ta = from + (wn + fr) * kRow + fo[kk], *tb = from + TN * kRow + (wm + fr) * kRow + fo[kk];
+#pragma unroll
+    for (int i = 0; i < kMi; ++i) fa[kk][i] = *(const uint4 *)(ta + 16 * kRow * i);
+#pragma unroll
+    for (int j = 0; j < kNi; ++j) fb[kk][j] = *(const uint4 *)(tb + 16 * kRow * j);
+  };
+  auto product = [&](int kk) {
+#pragma unroll
+    for (int i = 0; i < kMi; ++i)
+#pragma unroll
+      for (int j = 0; j < kNi; ++j) acc[i][j] = kp_mfma<HDT>(fa[kk][i], fb[kk][j], acc[i][j]);
+  };
+  auto fold = [&]() {
+#pragma unroll
+    for (int i = 0; i < kMi; ++i)
+#pragma unroll
+      for (int j = 0; j < kNi; ++j) {
+        sum[i][j] += acc[i][j];
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  };
+  // one step: its first half's operands are in registers; the second half's are read and step + 2 is staged
+  // under the first half's products, the next step's first half is read under the second's
+  uint8_t *cur = s_t, *nxt = s_t + kBuf, *free = s_t + 2 * kBuf;
+  auto step = [&](u32x4(&a)[kPa], u32x4(&b)[kPb], int i) {
+    read(1, cur);
+    __builtin_amdgcn_sched_barrier(0);
+    stage(a, b, free);  // step i + 2, into the buffer step i - 1 was read from
+    product(0);
+#pragma unroll
+    for (int g = 0; g < kPa + kPb; ++g) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product,
+      __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);  // a staging write
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    read(0, nxt);
+    fetch(a, b, i + 4);
+    product(1);
+#pragma unroll
+    for (int g = 0; g < kMi + kNi; ++g) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an operand read,
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product
+    }
+#pragma unroll
+    for (int g = 0; g < kPa + kPb; ++g) {
+      __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // a load,
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product
+    }
+    lds_barrier();
+    uint8_t *t = cur;
+    cur = nxt, nxt = free, free = t;
+  };
+  fetch(a0, b0, 0);
+  fetch(a1, b1, 1);
+  __builtin_amdgcn_sched_barrier(0);
+  stage(a0, b0, cur);
+  fetch(a0, b0, 2);
+  __builtin_amdgcn_sched_barrier(0);
+  stage(a1, b1, nxt);
+  fetch(a1, b1, 3);
+  lds_barrier();
+  read(0, cur);
+  int i = 0;
+  for (; i + 1 < steps; i += 2) {
+    step(a0, b0, i);
+    step(a1, b1, i + 1);
+    if ((i & (kGemmFold - 1)) == kGemmFold - 2) fold();
+  }
+  if (i < steps) step(a0, b0, i);
+  fold();
+
+  // bias, rounding to the h dtype (F.linear's output), RoPE, store: channels n .. n + 3 of token m (D and
+  // n are multiples of 4, so the four lie within a head and their angles are one vector)
+  constexpr int ODT = CS32 ? FFA_DT_F32 : HDT;
+  auto load4 = [](const void *p, size_t i, float *x) {
+    if constexpr (CS32) {
+      const float4 v = *(const float4 *)((const float *)p + i);
+      x[0] = v.x, x[1] = v.y, x[2] = v.z, x[3] = v.w;
+    } else {
+      const uint2 v = *(const uint2 *)((const uint16_t *)p + i);
+      const uint32_t b[4] = {v.x & 0xffffu, v.x >> 16, v.y & 0xffffu, v.y >> 16};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = HDT == FFA_DT_BF16 ? bf16_bits_to_f32(b[e]) : f16_bits_to_f32(b[e]);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < kMi; ++i) {
+    const int n = n0 + wn + 16 * i + 4 * fq;
+    if (n >= N) continue;
+    float bv[4] = {0.f, 0.f, 0.f, 0.f};
+    if (bias != nullptr)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bv[e] = load_any(bias, n + e, HDT);
+    const int d = n % D;
+#pragma unroll
+    for (int j = 0; j < kNi; ++j) {
+      const int m = m0 + wm + 16 * j + fr;
+      if (m >= M) continue;
+      float c[4], sn[4], o[4];
+      load4(cos, (size_t)(m % T) * D + d, c);
+      load4(sin, (size_t)(m % T) * D + d, sn);
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        const float x0 = round_to(sum[i][j][e] + bv[e], HDT), x1 = round_to(sum[i][j][e + 1] + bv[e + 1], HDT);
+        o[e] = rope_one(x0, x1, false, c[e], sn[e], ODT);
+        o[e + 1] = rope_one(x1, x0, true, c[e + 1], sn[e + 1], ODT);
+      }
+      const size_t at = (size_t)m * N + n;
+      if constexpr (CS32)
+        *(float4 *)((float *)kout + at) = make_float4(o[0], o[1], o[2], o[3]);
+      else if constexpr (HDT == FFA_DT_BF16)
+        *(uint2 *)((uint16_t *)kout + at) = make_uint2(f32_to_bf16_bits(o[0]) | (f32_to_bf16_bits(o[1]) << 16),
+                                                       f32_to_bf16_bits(o[2]) | (f32_to_bf16_bits(o[3]) << 16));
+      else
+        *(uint2 *)((uint16_t *)kout + at) = make_uint2(pk_f16_bits(o[0], o[1]), pk_f16_bits(o[2], o[3]));
+    }
+  }
+}
+
 // K-proj + RoPE (fp32 cos/sin rows per token) + g32 quantize + paged append; the 32 channels of a
 // workgroup are one g32 group of one KV head, so quantization needs no other workgroup.
 template <int HDT>
@@ -643,6 +837,45 @@ extern "C" int ffa_q2_quantize_channel(const void *k, int k_dtype, int B, int T,
                               (hipStream_t)stream);
 }
 
+template <int HDT, int TM, int TN>
+static void launch_kproj_tile(const void *h, const void *w, const void *bias, const void *cos, const void *sin, int csdt,
+                              int M, int T, int H, int N, int D, void *k_out, hipStream_t st) {
+  const dim3 grid((unsigned)((size_t)((N + TN - 1) / TN) * ((M + TM - 1) / TM)));
+  if (csdt == FFA_DT_F32)
+    hipLaunchKernelGGL((ffa::kproj_rope_tile_kernel<HDT, true, TM, TN>), grid, dim3(256), 0, st, h, w, bias, cos, sin, M,
+                       T, H, N, D, k_out);
+  else
+    hipLaunchKernelGGL((ffa::kproj_rope_tile_kernel<HDT, false, TM, TN>), grid, dim3(256), 0, st, h, w, bias, cos, sin, M,
+                       T, H, N, D, k_out);
+}
+
+template <int HDT>
+static void launch_kproj_rope(const void *h, const void *w, const void *bias, const void *cos, const void *sin, int csdt,
+                              int M, int T, int H, int N, int D, void *k_out, int odt, hipStream_t st) {
+  // The largest tile that still gives every CU a workgroup (us at H = 4096, N = 1024, bf16; the 16 x 32 tiles
+  // of kproj_rope_kernel last):
+  //   M = 4096   128x128 53, 128x64 57, 64x64 72, 249        M = 1024   64x64 22, 32x64 26, 128x64 30, 67
+  //   M = 2048   128x64 32, 64x64 36, 128x128 45, 128        M = 512    32x64 18, 64x64 20, 36
+  // 32x64 tiles pay from half the CUs on (M = 256: 17.6 against 19.3; M = 128: 16.8 against 10.9).
+  // Vector loads and stores need D and the pointers aligned, the K loop H a multiple of 64 (and a tile's rows
+  // within a buffer resource's 31 bits).
+  if (H % ffa::kGemmK == 0 && H < (1 << 22) && D % 4 == 0 && aligned(h, 16) && aligned(w, 16) && aligned(k_out, 16) &&
+      aligned(cos, 16) && aligned(sin, 16)) {
+    const int cus = ffa::device_cus() > 0 ? ffa::device_cus() : 256;
+    auto tiles = [&](int tm, int tn) { return (long)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
+    if (tiles(128, 128) >= cus)
+      return launch_kproj_tile<HDT, 128, 128>(h, w, bias, cos, sin, csdt, M, T, H, N, D, k_out, st);
+    if (tiles(128, 64) >= cus)
+      return launch_kproj_tile<HDT, 128, 64>(h, w, bias, cos, sin, csdt, M, T, H, N, D, k_out, st);
+    if (tiles(64, 64) >= cus)
+      return launch_kproj_tile<HDT, 64, 64>(h, w, bias, cos, sin, csdt, M, T, H, N, D, k_out, st);
+    if (tiles(32, 64) >= cus / 2)
+      return launch_kproj_tile<HDT, 32, 64>(h, w, bias, cos, sin, csdt, M, T, H, N, D, k_out, st);
+  }
+  hipLaunchKernelGGL(ffa::kproj_rope_kernel<HDT>, dim3((unsigned)((N / 32) * ((M + 15) / 16))), dim3(512), 0, st, h, w,
+                     bias, cos, sin, csdt, M, T, H, N, D, k_out, odt);
+}
+
 extern "C" int ffa_kproj_rope(const void *h, const void *w_k, const void *bias, int h_dtype, const void *cos,
                               const void *sin, int cs_dtype, int B, int T, int H, int HKV, int D, void *k_out,
                               void *stream) {
@@ -656,13 +889,10 @@ extern "C" int ffa_kproj_rope(const void *h, const void *w_k, const void *bias, 
   const int M = B * T, N = HKV * D;
   const int odt = cs_dtype == FFA_DT_F32 ? FFA_DT_F32 : h_dtype;
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid((unsigned)((N / 32) * ((M + 15) / 16)));
   if (h_dtype == FFA_DT_BF16)
-    hipLaunchKernelGGL(ffa::kproj_rope_kernel<FFA_DT_BF16>, grid, dim3(512), 0, st, h, w_k, bias, cos, sin, cs_dtype, M,
-                       T, H, N, D, k_out, odt);
+    launch_kproj_rope<FFA_DT_BF16>(h, w_k, bias, cos, sin, cs_dtype, M, T, H, N, D, k_out, odt, st);
   else
-    hipLaunchKernelGGL(ffa::kproj_rope_kernel<FFA_DT_F16>, grid, dim3(512), 0, st, h, w_k, bias, cos, sin, cs_dtype, M,
-                       T, H, N, D, k_out, odt);
+    launch_kproj_rope<FFA_DT_F16>(h, w_k, bias, cos, sin, cs_dtype, M, T, H, N, D, k_out, odt, st);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return ffa_set_error_internal(FFA_E_LAUNCH, hipGetErrorString(e));
   return FFA_OK;

@@ -121,3 +121,43 @@ def test_q2_quantizer_vector_route_equals_scalar_route(gpu, tau, B, T, HKV, D):
         a, b = quantize_per_channel(k, fp8), quantize_per_channel(_misaligned(k), fp8)
         for x, y in zip(a, b):
             assert np.array_equal(_u8(x), _u8(y))
+
+
+# ------------------------------------------------------------------- K projection + RoPE
+@pytest.mark.gpu
+@pytest.mark.parametrize("h_dt", ["bf16", "fp16"])
+@pytest.mark.parametrize("B,T,HKV,D,H,cs32,bias", [
+    (1, 4100, 8, 128, 64, True, False),    # 128 x 128 tiles (33 x 8), one K step, a ragged last row of tiles
+    (2, 2048, 8, 128, 576, False, True),   # 128 x 128, nine steps (a fold and an odd tail), two sequences
+    (1, 4200, 35, 32, 192, True, True),    # 128 x 128, a ragged last column of tiles, grid not a multiple of 8
+    (3, 700, 8, 128, 192, True, True),     # 128 x 64 (17 x 16)
+    (1, 1030, 8, 128, 1024, False, False), # 64 x 64 (17 x 16), two folds
+    (1, 290, 7, 128, 128, True, False),    # 32 x 64 (10 x 14)
+    (1, 300, 8, 96, 96, True, False),      # H no multiple of 64: the 16 x 32 kernel
+])
+def test_kproj_rope_tiles(gpu, h_dt, B, T, HKV, D, H, cs32, bias):
+    """Every tile size of the projection against fp64.  The projection is rounded to h's type from fp32 sums: equal
+    to the rounding of the fp64 product but where that lies within the sums' error of a rounding boundary, which
+    moves it by one ulp of h's type (2^-8 or 2^-11 relative, at most 2^-7 / 2^-10 of the pair through RoPE, and
+    one rounding more to a 16-bit result).  The sums' error is about 2^-22 of the terms' size: fewer than 1 in 100
+    elements can be so near."""
+    from ffa_mi355x import kfmt_quant as KQ
+
+    dt = TORCH_DT[h_dt]
+    g = torch.Generator().manual_seed(T)
+    h = torch.randn(B, T, H, generator=g).to(dt).to(gpu)
+    w = (torch.randn(HKV * D, H, generator=g) / H ** 0.5).to(dt).to(gpu)
+    bv = torch.randn(HKV * D, generator=g).to(dt).to(gpu) if bias else None
+    ang = torch.rand(T, D, generator=g) * 6.28
+    cos, sin = (x.to(torch.float32 if cs32 else dt).to(gpu) for x in (ang.cos(), ang.sin()))
+    k = KQ.kproj_rope(h, w, cos, sin, HKV, D, bias=bv)
+    lin = h.double() @ w.double().t().contiguous()
+    lin = (lin if bv is None else lin + bv.double()).to(dt).view(B, T, HKV, D)
+    rot = torch.stack((-lin[..., 1::2], lin[..., ::2]), -1).flatten(-2)
+    ref = lin * cos[None, :, None] + rot * sin[None, :, None]
+    assert k.dtype == ref.dtype
+    off = (k.double() - ref.double()).abs()
+    pair = lin.double().abs() + rot.double().abs()
+    ulp = 2.0 ** (-7 if h_dt == "bf16" else -10)
+    assert float((off > 0).float().mean()) < 1e-2
+    assert bool((off <= ulp * pair * (1 if cs32 else 2) + 1e-30).all())
