@@ -44,6 +44,12 @@ __device__ __forceinline__ uint32_t pk_f16_bits(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2));
 }
 
+// the same for bf16 (v_cvt_pk_bf16_f32: the bits of f32_to_bf16_bits for every input)
+__device__ __forceinline__ uint32_t pk_bf16_bits(float a, float b) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
+}
+
 // load element i of a float tensor of runtime dtype (0=f16, 1=bf16, 2=f32)
 __device__ __forceinline__ float load_any(const void *p, size_t i, int dt) {
   if (dt == 2) return ((const float *)p)[i];
@@ -148,8 +154,7 @@ __device__ __forceinline__ void round8(float *x) {
 #pragma unroll
     for (int e = 0; e < 8; e += 2) {
       if constexpr (DT == 1) {
-        typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-        const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){x[e], x[e + 1]}, bf16x2));
+        const uint32_t w = pk_bf16_bits(x[e], x[e + 1]);
         x[e] = __uint_as_float(w << 16);
         x[e + 1] = __uint_as_float(w & 0xffff0000u);
       } else {

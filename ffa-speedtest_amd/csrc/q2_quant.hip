@@ -673,71 +673,124 @@ __global__ __launch_bounds__(256) void q2_g32_append_kernel(const void *k, int k
 }
 
 
+// eight floats to eight consecutive elements of dtype DT in registers: one 16-byte word, or two (f32)
+template <int DT>
+__device__ __forceinline__ Raw8<DT> pack8(const float *x) {
+  Raw8<DT> r;
+  if constexpr (DT == 2) {
+    r.v[0] = make_uint4(__float_as_uint(x[0]), __float_as_uint(x[1]), __float_as_uint(x[2]), __float_as_uint(x[3]));
+    r.v[1] = make_uint4(__float_as_uint(x[4]), __float_as_uint(x[5]), __float_as_uint(x[6]), __float_as_uint(x[7]));
+  } else {
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = DT == 1 ? pk_bf16_bits(x[2 * e], x[2 * e + 1]) : pk_f16_bits(x[2 * e], x[2 * e + 1]);
+    r.v[0] = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+  return r;
+}
+
 // Paged g32 cache -> contiguous K and V (the exact-attention path of the HF integration, which the
 // reference feeds with dequantized keys: ffa-fp8fp8/e2e/fp8fp8_cache.py:60-69, returned by update at
 // :84-89).  One workgroup per (sequence, page of the sequence, KV head): K = c * s + z + r in fp32
-// (c * s is exact, so the fma rounds once, as the sum does), then one rounding to the output dtype;
-// V read from the V^T page through shared memory so that both outputs are written as rows.  Tokens at
-// or past the sequence's length are written as zeros; block-table entries outside the pool read page 0.
+// (c * s is exact, so the fma rounds once, as the sum does), then one rounding to the output dtype.
+// Tokens at or past the sequence's length are written as zeros; block-table entries outside the pool
+// read page 0.
+// Bound by the bytes (24 read, 27 KB or more written per page and head).  Everything is read in the
+// pool's own order, 1 KB a wave and load: wave tau, lane (group g, m) holds all 32 channels of group g of
+// token 4 m + tau (residual blocks (tau, 0) and (tau, 1)), and V^T pieces of 8 tokens of one column.
+// Rows are put together in LDS and written 16 bytes a lane, whole rows at a time; V is turned by the
+// transposing LDS read (4 tokens x 32 columns per 16 lanes).  Written 2 bytes a lane at 64-byte distances,
+// as K and V were before, the cache of 4 sequences of 3K to 8K tokens, 214 MB, took 300 us; 56 now.
+template <bool E4M3, int VDT, int ODT>
 __global__ __launch_bounds__(256) void q2_paged_dequant_kernel(const uint8_t *kq_pages, const uint16_t *s_pages,
                                                                const uint16_t *z_pages, const uint8_t *r_pages,
-                                                               int res_e4m3, const uint16_t *v_pages, int vdt,
-                                                               const int32_t *bt, int bt_stride, int num_pages,
-                                                               const int32_t *seq_lens, int T, int HKV, void *k_out,
-                                                               void *v_out, int odt) {
+                                                               const uint16_t *v_pages, const int32_t *bt, int bt_stride,
+                                                               int num_pages, const int32_t *seq_lens, int T, int HKV,
+                                                               void *k_out, void *v_out) {
   constexpr int D = 128;
+  constexpr int kEs = ODT == 2 ? 4 : 2, kRow = D * kEs, kPcs = kRow / 16;  // output row: bytes, 16-byte pieces
+  constexpr int kVPitch = 144;  // LDS bytes of a V^T column (64 tokens), 16 past 128 to spread the banks
+  constexpr int kLds = 64 * kRow > D * kVPitch ? 64 * kRow : D * kVPitch;
+  __shared__ __attribute__((aligned(16))) uint8_t s_t[kLds];
   const int j = blockIdx.x, hkv = blockIdx.y, b = blockIdx.z;
   const int Tb = seq_lens ? min(max(seq_lens[b], 0), T) : T;
+  const int nv = min(max(Tb - 64 * j, 0), 64);  // tokens of the page that the sequence holds
   int page = bt[(size_t)b * bt_stride + j];
   page = (unsigned)page < (unsigned)num_pages ? page : 0;
   const size_t blk = (size_t)page * HKV + hkv;
-  __shared__ uint16_t s_v[64][D + 2];
-  // V^T: 1024 16-byte pieces (8 tokens of one column); piece P holds column 16 (P >> 7) + (P & 15),
-  // tokens 16 ((P >> 4) & 3) + 8 ((P >> 6) & 1) + (0..7)
-  const uint4 *vp = (const uint4 *)(v_pages + blk * (D * 64));
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int P = threadIdx.x + 256 * i;
-    const int c = 16 * (P >> 7) + (P & 15), t0 = 16 * ((P >> 4) & 3) + 8 * ((P >> 6) & 1);
-    const uint4 w = vp[P];
-    const uint32_t e[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      s_v[t0 + 2 * k][c] = (uint16_t)(e[k] & 0xffffu);
-      s_v[t0 + 2 * k + 1][c] = (uint16_t)(e[k] >> 16);
-    }
-  }
-  // K: thread (token t, group g) dequantizes 32 channels
-  const int t = threadIdx.x >> 2, g = threadIdx.x & 3;
-  const int tok = 64 * j + t;
-  const bool valid = tok < Tb;
+  const int lane = threadIdx.x & 63, tau = threadIdx.x >> 6;
+  const int m = lane & 15, g = lane >> 4, t = 4 * m + tau;
   const uint2 cw = *(const uint2 *)(kq_pages + blk * (4 * 64 * 8) + codes_off(g, t));
   const int ss = 16 * (t >> 4) + 4 * (t & 3) + ((t >> 2) & 3);  // tile-major scale slot, as appended
   const float sc = f16_bits_to_f32(s_pages[blk * (4 * 64) + gscale_off(g, ss)]);
   const float zr = f16_bits_to_f32(z_pages[blk * (4 * 64) + gscale_off(g, ss)]);
-  const uint4 r0 = *(const uint4 *)(r_pages + blk * (64 * D) + res_off(t, 32 * g));
-  const uint4 r1 = *(const uint4 *)(r_pages + blk * (64 * D) + res_off(t, 32 * g + 16));
+  const uint4 *rp = (const uint4 *)(r_pages + blk * (64 * D)) + tau * 128 + lane;
+  const uint4 r0 = rp[0], r1 = rp[64];
+  // V^T: 1024 16-byte pieces (8 tokens of one column); piece P holds column 16 (P >> 7) + (P & 15),
+  // tokens 16 ((P >> 4) & 3) + 8 ((P >> 6) & 1) + (0..7)
+  const uint4 *vp = (const uint4 *)(v_pages + blk * (D * 64));
+  uint4 vw[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) vw[i] = vp[threadIdx.x + 256 * i];
+
   const uint32_t rw[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
   const uint32_t cwords[2] = {cw.x, cw.y};
-  const size_t orow = ((size_t)b * T + tok) * HKV + hkv;
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const f16x8 rv = res_e4m3 ? fp8x8_to_f16x8<kResE4M3>(rw[2 * a], rw[2 * a + 1])
-                              : fp8x8_to_f16x8<kResE5M2>(rw[2 * a], rw[2 * a + 1]);  // exact
+  for (int a = 0; a < 4; ++a) {  // channels 32 g + 8 a + (0..7)
+    const f16x8 rv = fp8x8_to_f16x8<E4M3 ? kResE4M3 : kResE5M2>(rw[2 * a], rw[2 * a + 1]);  // exact
+    float k[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      const int i = 8 * a + e;
-      const uint32_t code = (cwords[i >> 4] >> (2 * (i & 15))) & 3u;
-      const float k = __builtin_fmaf((float)code, sc, zr) + (float)rv[e];
-      store_any(k_out, orow * D + 32 * g + i, odt, valid ? k : 0.f);
+      const uint32_t code = (cwords[a >> 1] >> (2 * ((8 * a + e) & 15))) & 3u;
+      const float x = __builtin_fmaf((float)code, sc, zr) + (float)rv[e];
+      k[e] = t < nv ? x : 0.f;
+    }
+    const Raw8<ODT> o = pack8<ODT>(k);
+    // piece q of row t at q ^ (m & 7): the 16 rows that a write touches start at different banks
+#pragma unroll
+    for (int h = 0; h < kEs / 2; ++h) {
+      const int q = (kPcs / 4) * g + (kEs / 2) * a + h;
+      *(uint4 *)(s_t + t * kRow + ((q ^ (m & 7)) * 16)) = o.v[h];
     }
   }
   __syncthreads();
+  const size_t orow = ((size_t)b * T + 64 * j) * HKV + hkv;  // row of the page's token 0
 #pragma unroll
-  for (int i = 0; i < 32; ++i) {
-    const uint32_t bits = s_v[t][32 * g + i];
-    const float x = vdt == FFA_DT_BF16 ? bf16_bits_to_f32(bits) : f16_bits_to_f32(bits);
-    store_any(v_out, orow * D + 32 * g + i, odt, valid ? x : 0.f);
+  for (int i = 0; i < 64 * kPcs / 256; ++i) {
+    const int tk = (threadIdx.x + 256 * i) / kPcs, q = threadIdx.x & (kPcs - 1);
+    const uint4 w = *(const uint4 *)(s_t + tk * kRow + ((q ^ ((tk >> 2) & 7)) * 16));
+    *(uint4 *)((uint8_t *)k_out + (orow + (size_t)tk * HKV) * kRow + 16 * q) = w;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int P = threadIdx.x + 256 * i;
+    const int c = 16 * (P >> 7) + (P & 15), t0 = 16 * ((P >> 4) & 3) + 8 * ((P >> 6) & 1);
+    *(uint4 *)(s_t + c * kVPitch + 2 * t0) = vw[i];
+  }
+  __syncthreads();
+  // lane x of a 16-lane group addresses 4 tokens of column 32 grp + 8 (x % 4) + x / 4 and receives, of token
+  // x % 4 of those, the columns that lanes x / 4 + 4 e address: 32 grp + 8 (x / 4) + e (e = 0..3); a second read
+  // 4 columns on completes its 8
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  const int x = lane & 15, col = 32 * g + 8 * (x & 3) + (x >> 2);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int tk0 = 16 * tau + 4 * i, tk = tk0 + (x & 3);
+    const auto *p0 = (const lds_s16x4 *)((__attribute__((address_space(3))) const uint8_t *)s_t + col * kVPitch + 2 * tk0);
+    const auto *p1 = (const lds_s16x4 *)((__attribute__((address_space(3))) const uint8_t *)s_t + (col + 4) * kVPitch + 2 * tk0);
+    const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)p0));
+    const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)p1));
+    Raw8<VDT> in;
+    in.v[0] = make_uint4(lo[0], lo[1], hi[0], hi[1]);
+    float v[8];
+    raw8_to_f32<VDT>(in, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = tk < nv ? v[e] : 0.f;
+    const Raw8<ODT> o = pack8<ODT>(v);
+#pragma unroll
+    for (int h = 0; h < kEs / 2; ++h)
+      *(uint4 *)((uint8_t *)v_out + (orow + (size_t)tk * HKV) * kRow + (32 * g + 8 * (x >> 2)) * kEs + 16 * h) = o.v[h];
   }
 }
 }  // namespace ffa
@@ -977,11 +1030,19 @@ extern "C" int ffa_q2_paged_dequant(const uint8_t *k_q_pages, const void *scale_
   if (!k_q_pages || !scale_pages || !zero_pages || !res_pages || !v_pages || !block_table || !k_out || !v_out)
     return ffa_set_error_internal(FFA_E_INVALID, "null pointer");
   if (T % ffa::kPage) return ffa_set_error_internal(FFA_E_INVALID, "T must be a multiple of the 64-token page");
-  hipLaunchKernelGGL(ffa::q2_paged_dequant_kernel, dim3((unsigned)(T / ffa::kPage), (unsigned)HKV, (unsigned)B),
-                     dim3(256), 0, (hipStream_t)stream, k_q_pages, (const uint16_t *)scale_pages,
-                     (const uint16_t *)zero_pages, res_pages, res_dtype == FFA_DT_FP8_E4M3 ? 1 : 0,
-                     (const uint16_t *)v_pages, v_dtype, block_table, bt_stride, num_pages, seq_lens, T, HKV, k_out,
-                     v_out, out_dtype);
+  const dim3 grid((unsigned)(T / ffa::kPage), (unsigned)HKV, (unsigned)B);
+#define FFA_CASE(EE, VV, OO)                                                                                         \
+  if ((res_dtype == FFA_DT_FP8_E4M3) == EE && v_dtype == VV && out_dtype == OO)                                      \
+    hipLaunchKernelGGL((ffa::q2_paged_dequant_kernel<EE, VV, OO>), grid, dim3(256), 0, (hipStream_t)stream,          \
+                       k_q_pages, (const uint16_t *)scale_pages, (const uint16_t *)zero_pages, res_pages,            \
+                       (const uint16_t *)v_pages, block_table, bt_stride, num_pages, seq_lens, T, HKV, k_out, v_out);
+#define FFA_CASES(EE, VV) FFA_CASE(EE, VV, FFA_DT_F16) FFA_CASE(EE, VV, FFA_DT_BF16) FFA_CASE(EE, VV, FFA_DT_F32)
+  FFA_CASES(true, FFA_DT_F16)
+  FFA_CASES(true, FFA_DT_BF16)
+  FFA_CASES(false, FFA_DT_F16)
+  FFA_CASES(false, FFA_DT_BF16)
+#undef FFA_CASES
+#undef FFA_CASE
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? FFA_OK : ffa_set_error_internal(FFA_E_LAUNCH, hipGetErrorString(e));
 }

@@ -161,3 +161,37 @@ def test_kproj_rope_tiles(gpu, h_dt, B, T, HKV, D, H, cs32, bias):
     ulp = 2.0 ** (-7 if h_dt == "bf16" else -10)
     assert float((off > 0).float().mean()) < 1e-2
     assert bool((off <= ulp * pair * (1 if cs32 else 2) + 1e-30).all())
+
+
+# ------------------------------------------------------------------- paged cache -> contiguous
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["e4m3fn", "e5m2"])
+@pytest.mark.parametrize("v_dt", ["fp16", "bf16"])
+def test_paged_dequantize_every_type(gpu, fmt, v_dt):
+    """Every residual, V and output type, lengths at page edges (0, 1, 63, 64, 65 tokens of the last page): fp32
+    fma(code, scale, zero) + residual of the pool's own bytes, rounded once."""
+    from ffa_mi355x.paged import CODES_ORDER, GSCALE_ORDER, RES_ORDER, VT_ORDER, PagedQ2Cache, scale_pos, to_logical
+
+    lens = [192, 129, 127, 65, 64, 1, 0]
+    B, HKV, npg = len(lens), 3, 3
+    g = torch.Generator().manual_seed(4)
+    cache = PagedQ2Cache(B * npg, HKV, gpu, res_dtype=FP8_DT[fmt], v_dtype=TORCH_DT[v_dt])
+    bt = torch.randperm(B * npg, generator=g).view(B, npg).int()
+    k, v = (torch.randn(B, 192, HKV, 128, generator=g).to(gpu) for _ in range(2))
+    cache.append(k, v, torch.zeros(B, dtype=torch.int32, device=gpu), bt.to(gpu))
+    codes = to_logical(cache.k_q.cpu().numpy(), CODES_ORDER, 8)  # [P, H, 4, 64, 8]
+    bits = (codes[..., None] >> np.array([0, 2, 4, 6], np.uint8)) & 3
+    c = bits.reshape(codes.shape[:-1] + (32,)).transpose(0, 1, 3, 2, 4).astype(np.float32)  # [P, H, 64, 4, 32]
+    sz = [to_logical(x.cpu().numpy(), GSCALE_ORDER)[..., scale_pos(np.arange(64))].transpose(0, 1, 3, 2)[..., None]
+          .astype(np.float32) for x in (cache.k_scale, cache.k_zero)]
+    res = to_logical(_u8(cache.k_res), RES_ORDER).reshape(c.shape)
+    rf = torch.from_numpy(res).view(FP8_DT[fmt]).float().numpy()
+    kf = torch.from_numpy(((c * sz[0] + sz[1]) + rf).reshape(B * npg, HKV, 64, 128))  # c * s is exact
+    vf = torch.from_numpy(to_logical(cache.v.view(torch.int16).cpu().numpy(), VT_ORDER)).view(TORCH_DT[v_dt]).float()
+    keep = (torch.arange(192)[None] < torch.tensor(lens)[:, None])[..., None, None]
+    want = [x.view(B, npg, HKV, 64, 128).permute(0, 1, 3, 2, 4).reshape(B, 192, HKV, 128) * keep
+            for x in (kf[bt.long()], vf.transpose(-1, -2)[bt.long()])]
+    for out in (torch.float32, torch.float16, torch.bfloat16):
+        got = cache.dequantize(bt.to(gpu), 192, torch.tensor(lens, dtype=torch.int32), out_dtype=out)
+        for x, y in zip(got, want):
+            assert torch.equal(x.cpu(), y.to(out))
