@@ -13,6 +13,7 @@
 #include "decode_common.h"
 #include "ffa_common.h"
 #include "ffa_mi355x.h"
+#include "page_tile.h"
 
 #include <stdio.h>
 
@@ -673,6 +674,53 @@ __global__ __launch_bounds__(256) void q2_g32_append_kernel(const void *k, int k
 }
 
 
+// The same append for many tokens, a (page, KV head) block per workgroup (page_tile.h): a thread holds a whole
+// 32-channel group, so extrema, scale, codes and residual are its own; codes by the scale's turning points
+// (q2_turn, of the fp32 quotient) instead of 32 divisions.  grid (KV head, tile, sequence).
+template <int KDT, bool E4M3>
+__global__ __launch_bounds__(256) void q2_g32_page_kernel(const void *k, int Tn, int HKV, const int32_t *pos,
+                                                          const int32_t *bt, int bt_stride, int num_pages,
+                                                          uint8_t *kq_pages, uint16_t *s_pages, uint16_t *z_pages,
+                                                          uint8_t *r_pages, const void *v_new, int vmode, void *v_pages) {
+  __shared__ __attribute__((aligned(16))) uint8_t s_t[page_tile_lds<KDT>()];
+  const int hkv = blockIdx.x, b = blockIdx.z;
+  const PageTile pt = page_tile(pos, bt, bt_stride, num_pages, b, blockIdx.y, Tn);
+  if (pt.page < 0) return;  // the whole workgroup
+  const size_t row0 = (size_t)b * Tn * HKV + hkv, blk = (size_t)pt.page * HKV + hkv;
+  float x[32];
+  page_tile_k<KDT>(k, row0, HKV, pt, s_t, x);
+  const int m = threadIdx.x & 15, g = (threadIdx.x >> 4) & 3, tau = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int t = 4 * m + tau;
+  float mn = x[0], mx = x[0];
+#pragma unroll
+  for (int e = 1; e < 32; ++e) mn = fminf(mn, x[e]), mx = fmaxf(mx, x[e]);
+  const float zr = (float)(_Float16)mn;
+  const float sc = (float)(_Float16)__fdiv_rn(fmaxf(mx - zr, 1e-6f), 3.0f);
+  const float t1 = q2_turn<FFA_DT_F32>(sc, 0), t2 = q2_turn<FFA_DT_F32>(sc, 1), t3 = q2_turn<FFA_DT_F32>(sc, 2);
+  uint32_t cw[2] = {0u, 0u};
+#pragma unroll
+  for (int e = 0; e < 32; ++e) {
+    const float y = x[e] - zr;
+    const uint32_t cq = y >= t3 ? 3u : (y >= t2 ? 2u : (y >= t1 ? 1u : 0u));
+    cw[e >> 4] |= cq << (2 * (e & 15));
+    x[e] -= (float)cq * sc + zr;
+  }
+  if (t >= pt.lo && t < pt.hi) {
+    uint4 *rp = (uint4 *)(r_pages + blk * (64 * 128)) + tau * 128 + lane;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint2 r0 = f32x8_to_fp8<E4M3>(x + 16 * h), r1 = f32x8_to_fp8<E4M3>(x + 16 * h + 8);
+      rp[64 * h] = make_uint4(r0.x, r0.y, r1.x, r1.y);
+    }
+    *(uint2 *)(kq_pages + blk * (4 * 64 * 8) + codes_off(g, t)) = make_uint2(cw[0], cw[1]);
+    const int ss = 16 * (t >> 4) + 4 * (t & 3) + ((t >> 2) & 3);  // tile-major scale slot
+    const size_t so = blk * (4 * 64) + gscale_off(g, ss);
+    s_pages[so] = (uint16_t)f32_to_f16_bits(sc);
+    z_pages[so] = (uint16_t)f32_to_f16_bits(zr);
+  }
+  if (v_new != nullptr) page_tile_v(v_new, vmode, row0, HKV, pt, s_t, (uint16_t *)v_pages + blk * (128 * 64));
+}
+
 // eight floats to eight consecutive elements of dtype DT in registers: one 16-byte word, or two (f32)
 template <int DT>
 __device__ __forceinline__ Raw8<DT> pack8(const float *x) {
@@ -1005,11 +1053,32 @@ extern "C" int ffa_q2_quantize_g32_append(const void *k, int k_dtype, int B, int
   if (!(k_dtype >= FFA_DT_F16 && k_dtype <= FFA_DT_F32)) return ffa_set_error_internal(FFA_E_INVALID, "k dtype");
   if (!(res_dtype == FFA_DT_FP8_E4M3 || res_dtype == FFA_DT_FP8_E5M2))
     return ffa_set_error_internal(FFA_E_INVALID, "residual dtype must be fp8");
-  const size_t rows = (size_t)B * Tn * HKV;
-  hipLaunchKernelGGL(ffa::q2_g32_append_kernel, dim3((unsigned)((rows + 1) / 2)), dim3(256), 0,
-                     (hipStream_t)stream, k, k_dtype, B * Tn, Tn, HKV, pos, block_table, bt_stride, num_pages, k_q_pages,
-                     (uint16_t *)scale_pages, (uint16_t *)zero_pages, res_pages, res_dtype == FFA_DT_FP8_E4M3 ? 1 : 0,
-                     v_new, v_pages);
+  const bool e4m3 = res_dtype == FFA_DT_FP8_E4M3;
+  // Whole pages from 32 tokens a sequence and 1024 in all (16K tokens of one sequence 29 us against 120, 4096
+  // 10 against 30, 512 equal, 16 x 32 tokens 6.5 against 6.0, one token of 64 sequences 6.4 against 3.6); the
+  // pieces need aligned rows and pools, the tiles are a grid dimension
+  if (Tn >= 32 && (long)B * Tn >= 1024 && ffa::page_tiles(Tn) <= 65535 && B <= 65535 && aligned(k, 16) &&
+      aligned(v_new, 16) && aligned(res_pages, 16) && aligned(v_pages, 16) && aligned(k_q_pages, 8)) {
+    const dim3 grid((unsigned)HKV, (unsigned)ffa::page_tiles(Tn), (unsigned)B);
+#define FFA_CASE(KK, EE)                                                                                            \
+  if (k_dtype == KK && e4m3 == EE)                                                                                  \
+    hipLaunchKernelGGL((ffa::q2_g32_page_kernel<KK, EE>), grid, dim3(256), 0, (hipStream_t)stream, k, Tn, HKV, pos, \
+                       block_table, bt_stride, num_pages, k_q_pages, (uint16_t *)scale_pages, (uint16_t *)zero_pages, \
+                       res_pages, v_new, ffa::kVSame, v_pages);
+    FFA_CASE(FFA_DT_F16, true)
+    FFA_CASE(FFA_DT_F16, false)
+    FFA_CASE(FFA_DT_BF16, true)
+    FFA_CASE(FFA_DT_BF16, false)
+    FFA_CASE(FFA_DT_F32, true)
+    FFA_CASE(FFA_DT_F32, false)
+#undef FFA_CASE
+  } else {
+    const size_t rows = (size_t)B * Tn * HKV;
+    hipLaunchKernelGGL(ffa::q2_g32_append_kernel, dim3((unsigned)((rows + 1) / 2)), dim3(256), 0,
+                       (hipStream_t)stream, k, k_dtype, B * Tn, Tn, HKV, pos, block_table, bt_stride, num_pages,
+                       k_q_pages, (uint16_t *)scale_pages, (uint16_t *)zero_pages, res_pages, e4m3 ? 1 : 0, v_new,
+                       v_pages);
+  }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return ffa_set_error_internal(FFA_E_LAUNCH, hipGetErrorString(e));
   return FFA_OK;

@@ -195,3 +195,48 @@ def test_paged_dequantize_every_type(gpu, fmt, v_dt):
         got = cache.dequantize(bt.to(gpu), 192, torch.tensor(lens, dtype=torch.int32), out_dtype=out)
         for x, y in zip(got, want):
             assert torch.equal(x.cpu(), y.to(out))
+
+
+# ------------------------------------------------------------------- paged appends
+def _pools(fmt, P, HKV, gpu, fill):
+    """A cache whose bytes start as given, and its pools as bytes."""
+    from ffa_mi355x.paged import PagedQ2Cache
+    from ffa_mi355x.paged_kfmt import PagedKfmtCache
+
+    c = PagedQ2Cache(P, HKV, gpu) if fmt == "q2" else PagedKfmtCache(fmt, P, HKV, gpu)
+    pools = [c.k_q, c.k_scale, c.k_zero, c.k_res, c.v] if fmt == "q2" else [c.k, c.k_scale, c.k_res, c.v]
+    for t in pools:
+        t.view(torch.uint8).fill_(fill)
+    return c, pools
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["q2"])
+@pytest.mark.parametrize("k_dt", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("B,Tn,HKV,pos", [
+    (1, 1024, 2, [0]),                    # whole pages
+    (1, 1100, 3, [63]),                   # one slot of the first page, a ragged last page
+    (2, 1025, 1, [1, 127]),
+    (33, 32, 2, [7 * i for i in range(33)]),  # half a page each, across a page edge for some
+])
+def test_page_append_equals_token_append(gpu, fmt, k_dt, B, Tn, HKV, pos):
+    """Appending whole pages writes the bytes that appending 31 tokens at a time (the per-token kernel) writes, and
+    leaves every other byte of the pools as it was; infinities, NaNs, zero and constant groups among the keys."""
+    g = torch.Generator().manual_seed(Tn)
+    npg = (max(pos) + Tn + 63) // 64 + 1
+    k = (torch.randn(B, Tn, HKV, 128, generator=g) * 2).to(TORCH_DT[k_dt])
+    k[0, 3, 0, :32], k[0, 4, 0, 32:64] = 0.0, 1.5
+    k[0, 5, 0, 7], k[0, 6, 0, 70], k[0, 7, 0, 100] = float("inf"), float("nan"), float("-inf")
+    k[0, 8, 0, :64], k[0, 9, 0, :64] = 1e-7, torch.linspace(-6e4, 6e4, 64).to(k.dtype)
+    k = k.to(gpu)
+    v = torch.randn(B, Tn, HKV, 128, generator=g).to(torch.float16).to(gpu)
+    bt = torch.randperm(B * npg, generator=g).view(B, npg).int().to(gpu)
+    p = torch.tensor(pos, dtype=torch.int32, device=gpu)
+    whole, wp = _pools(fmt, B * npg, HKV, gpu, 0x5A)
+    parts, pp = _pools(fmt, B * npg, HKV, gpu, 0x5A)
+    whole.append(k, v, p, bt)
+    for n in range(0, Tn, 31):
+        parts.append(k[:, n:n + 31].contiguous(), v[:, n:n + 31].contiguous(), p + n, bt)
+    for x, y in zip(wp, pp):
+        assert np.array_equal(_u8(x), _u8(y))
+    assert any((_u8(x) != 0x5A).any() for x in wp)
