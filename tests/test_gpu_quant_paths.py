@@ -210,24 +210,61 @@ def _pools(fmt, P, HKV, gpu, fill):
     return c, pools
 
 
+def _odd_groups(k):
+    """Zero, constant, tiny and wide groups, infinities and NaNs among the keys [B, T, H, 128]."""
+    k[0, 3, 0, :32], k[0, 4, 0, 32:64] = 0.0, 1.5
+    k[0, 5, 0, 7], k[0, 6, 0, 70], k[0, 7, 0, 100] = float("inf"), float("nan"), float("-inf")
+    k[0, 8, 0, :64], k[0, 9, 0, :64] = 1e-7, torch.linspace(-6e4, 6e4, 64).to(k.dtype)
+    if k.dtype != torch.float16:
+        k[0, 2, 0, :32] = 1e38
+        k[0, 2, 0, 32:64] = torch.linspace(-1e38, 1e38, 32).to(k.dtype)
+        k[0, 1, 0, :] = torch.linspace(-1e-44, 1e-44, 128).to(k.dtype)
+        k[0, 1, 0, 5], k[0, 1, 0, 70] = 300.0, -2600.0
+
+
+def test_nvfp4_and_nf4_code_turning_points():
+    """The float that |k| (nvfp4) or k (nf4) has to reach for the next code equals where fl32(k / scale) passes the
+    midpoint, for every e4m3 scale and a sample of fp16 / fp32 ones, seven floats to each side."""
+    e4 = torch.arange(1, 0x7F, dtype=torch.uint8).view(torch.float8_e4m3fn).float()
+    for c in (0.25, 0.75, 1.25, 1.75, 2.5, 3.5, 5.0):
+        for n in range(-7, 8):
+            x = ((e4 * c).view(torch.int32) + n).view(torch.float32)
+            assert torch.equal(x >= e4 * c, x / e4 >= c)
+    book = torch.from_numpy(OF.NF4_CODEBOOK)
+    mids = (book[:-1] + book[1:]) * 0.5
+    g = torch.Generator().manual_seed(3)
+    sc = torch.cat([torch.arange(17, 0x7C00, 7, dtype=torch.int16).view(torch.float16).float(),
+                    torch.rand(5000, generator=g) * torch.exp2(torch.randint(-18, 60, (5000,), generator=g).float())])
+    sc = sc[sc >= 1e-6]
+    for mid in mids:
+        up = torch.nextafter(mid, torch.tensor(1.0))
+        v = sc.double() * (0.5 * (mid.double() + up.double()))
+        t = v.float()
+        odd = bool(mid.view(torch.int32) & 1)
+        t = torch.where(t.double() < v if odd else t.double() <= v, torch.nextafter(t, torch.full_like(t, 1e38)), t)
+        for n in range(-7, 8):
+            x = (t.view(torch.int32) + n).view(torch.float32)
+            assert torch.equal(x >= t, x / sc > mid)
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("fmt", ["q2"])
+@pytest.mark.parametrize("fmt", ["q2", "nvfp4", "nf4"])
 @pytest.mark.parametrize("k_dt", ["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("B,Tn,HKV,pos", [
     (1, 1024, 2, [0]),                    # whole pages
     (1, 1100, 3, [63]),                   # one slot of the first page, a ragged last page
     (2, 1025, 1, [1, 127]),
     (33, 32, 2, [7 * i for i in range(33)]),  # half a page each, across a page edge for some
+    (5, 1, 2, [0, 1, 63, 64, 130]),       # single tokens (whole pages for the 4-bit formats only)
 ])
 def test_page_append_equals_token_append(gpu, fmt, k_dt, B, Tn, HKV, pos):
-    """Appending whole pages writes the bytes that appending 31 tokens at a time (the per-token kernel) writes, and
+    """Appending whole pages writes the bytes that the per-token kernel (which takes keys at any address) writes, and
     leaves every other byte of the pools as it was; infinities, NaNs, zero and constant groups among the keys."""
     g = torch.Generator().manual_seed(Tn)
     npg = (max(pos) + Tn + 63) // 64 + 1
     k = (torch.randn(B, Tn, HKV, 128, generator=g) * 2).to(TORCH_DT[k_dt])
-    k[0, 3, 0, :32], k[0, 4, 0, 32:64] = 0.0, 1.5
-    k[0, 5, 0, 7], k[0, 6, 0, 70], k[0, 7, 0, 100] = float("inf"), float("nan"), float("-inf")
-    k[0, 8, 0, :64], k[0, 9, 0, :64] = 1e-7, torch.linspace(-6e4, 6e4, 64).to(k.dtype)
+    if Tn > 9:
+        _odd_groups(k)
     k = k.to(gpu)
     v = torch.randn(B, Tn, HKV, 128, generator=g).to(torch.float16).to(gpu)
     bt = torch.randperm(B * npg, generator=g).view(B, npg).int().to(gpu)
@@ -235,8 +272,7 @@ def test_page_append_equals_token_append(gpu, fmt, k_dt, B, Tn, HKV, pos):
     whole, wp = _pools(fmt, B * npg, HKV, gpu, 0x5A)
     parts, pp = _pools(fmt, B * npg, HKV, gpu, 0x5A)
     whole.append(k, v, p, bt)
-    for n in range(0, Tn, 31):
-        parts.append(k[:, n:n + 31].contiguous(), v[:, n:n + 31].contiguous(), p + n, bt)
+    parts.append(_misaligned(k), v, p, bt)
     for x, y in zip(wp, pp):
         assert np.array_equal(_u8(x), _u8(y))
     assert any((_u8(x) != 0x5A).any() for x in wp)
