@@ -141,6 +141,121 @@ __global__ __launch_bounds__(256) void nvfp4_quant_kernel(const void *k, int kdt
   }
 }
 
+// values of eight e2m1 codes (low nibble first), exact
+__device__ __forceinline__ void fp4_levels8(uint32_t w, float *l) {
+  const f32x2 a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0), b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1);
+  const f32x2 c = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 2), d = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 3);
+  l[0] = a[0], l[1] = a[1], l[2] = b[0], l[3] = b[1], l[4] = c[0], l[5] = c[1], l[6] = d[0], l[7] = d[1];
+}
+
+// The same over vectors of 8 channels (D a multiple of 8, aligned pointers).  A page's K is read once: up to
+// kHold vectors a thread stay in registers from the maximum to the codes (a page of 128 tokens x 128 channels
+// in 16 bits), longer pages are read again.  The codes come by comparison: the scale is one value for the whole
+// workgroup, so where tau(|k| / scale) passes an e2m1 midpoint is seven floats, worked out once (fp4_turn), in
+// place of a division and a rounding per element.  Bound by the bytes then; element by element, with integer
+// divisions for the indices, a call on 20K x 1024 bf16 keys (72 MB) took 104 us; now 25.
+//
+// Smallest float that |k| has to reach: tau(fl32(|k| / sc)) >= c for a midpoint c of the e2m1 levels.  c is an
+// even value of every tau here, so the quotient has to reach the middle of c and the tau value below it, q.  sc *
+// q is exact in double; for 16-bit k and sc, k / sc is q or further than an fp32 rounding from it.  An infinite
+// scale takes code 0 (x / inf = 0, inf / inf = NaN): no float reaches a NaN.
+template <int KDT>
+__device__ __forceinline__ float fp4_turn(float sc, float c) {
+  constexpr int p = KDT == 2 ? 24 : (KDT == 1 ? 8 : 11);  // significant bits of tau
+  const float below = c == 0.25f ? 0.125f : (c < 1.f ? 0.5f : (c < 2.f ? 1.f : (c < 4.f ? 2.f : 4.f)));  // its binade
+  const double v = (double)sc * ((double)c - (double)below * (1.0 / (double)(1u << p)));
+  float f = (float)v;
+  if ((double)f < v) f = __uint_as_float(__float_as_uint(f) + 1u);
+  return sc < INFINITY ? f : __builtin_nanf("");
+}
+// |k| up to which tau(fl32(|k| / sc)) is zero (its sign is then not a code's): sc times half the least tau value
+template <int KDT>
+__device__ __forceinline__ float fp4_zero(float sc) {
+  if constexpr (KDT == 0) return sc * 0x1p-25f;
+  else if constexpr (KDT == 1) return sc * 0x1p-134f;  // inexact only below every bf16 value
+  else return sc < 0x1p25f ? __uint_as_float((uint32_t)(sc * 0.5f)) : sc * 0x1p-75f * 0x1p-75f;  // in units of 2^-149
+}
+
+template <int KDT, bool E4M3>
+__global__ __launch_bounds__(256) void nvfp4_quant8_kernel(const void *k, int T, int HKV, int D, int page, uint8_t *packed,
+                                                           void *scale, uint8_t *res) {
+  constexpr int kHold = KDT == 2 ? 4 : 8;
+  const int hkv = blockIdx.x, pg = blockIdx.y, b = blockIdx.z, npg = gridDim.y;
+  const int t0 = pg * page, nt = min(page, T - t0), per = D / 8, items = nt * per;
+  auto row_of = [&](int i) { return ((size_t)b * T + t0 + i / per) * HKV + hkv; };
+  float mx = 0.f;
+  Raw8<KDT> w[kHold];
+  for (int i0 = threadIdx.x; i0 < items; i0 += 256 * kHold) {
+#pragma unroll
+    for (int u = 0; u < kHold; ++u) {  // vectors past the page repeat its last: no effect on the maximum
+      const int i = min(i0 + 256 * u, items - 1);
+      w[u] = load8<KDT>(k, row_of(i) * D + 8 * (i % per));
+    }
+#pragma unroll
+    for (int u = 0; u < kHold; ++u) {
+      float x[8];
+      raw8_to_f32<KDT>(w[u], x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(x[e]));
+    }
+  }
+  mx = wave_max(mx);
+  __shared__ float s_red[4];
+  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
+  // scale = (amax / 6).clamp_min(1e-6), both in tau
+  const float sc = fmaxf(round_to(__fdiv_rn(mx, 6.0f), KDT), round_to(1e-6f, KDT));
+  if (threadIdx.x == 0) store_any(scale, ((size_t)b * npg + pg) * HKV + hkv, KDT, sc);
+  const float mid[7] = {0.25f, 0.75f, 1.25f, 1.75f, 2.5f, 3.5f, 5.0f};
+  float turn[7];
+#pragma unroll
+  for (int j = 0; j < 7; ++j) turn[j] = fp4_turn<KDT>(sc, mid[j]);
+  const float zero = fp4_zero<KDT>(sc);
+  const bool held = items <= 256 * kHold;
+  for (int i0 = threadIdx.x; i0 < items; i0 += 256 * kHold) {
+    if (!held) {
+#pragma unroll
+      for (int u = 0; u < kHold; ++u) {
+        const int i = min(i0 + 256 * u, items - 1);
+        w[u] = load8<KDT>(k, row_of(i) * D + 8 * (i % per));
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kHold; ++u) {
+      const int i = i0 + 256 * u;
+      if (i >= items) break;
+      float x[8], d[8];
+      raw8_to_f32<KDT>(w[u], x);
+      uint32_t cw = 0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float ax = fabsf(x[e]);
+        uint32_t c = 0;
+#pragma unroll
+        for (int j = 0; j < 7; ++j) c += ax >= turn[j] ? 1u : 0u;
+        cw |= (c | (x[e] < 0.f && ax > zero ? 8u : 0u)) << (4 * e);
+      }
+      fp4_levels8(cw, d);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) d[e] *= sc;
+      round8<KDT>(d);  // +-level * s in tau
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        // separate values: the compiler would pair the subtractions between two fp16 roundings and then find no
+        // instruction for the pair
+        if constexpr (KDT == 0) asm("" : "+v"(d[e]));
+        d[e] = x[e] - d[e];
+      }
+      round8<KDT>(d);  // k - that in tau
+      const size_t row = row_of(i);
+      const int c8 = i % per;
+      *(uint2 *)(res + row * D + 8 * c8) = f32x8_to_fp8<E4M3>(d);
+      *(uint32_t *)(packed + row * (D / 2) + 4 * c8) = cw;
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // nf4: per-channel absmax over T (splits, then a final pass), then codes
 // ---------------------------------------------------------------------------
@@ -398,11 +513,10 @@ __global__ __launch_bounds__(256) void kfmt_page_append_kernel(const void *k, in
       }
 #pragma unroll
       for (int e = 16 * h; e < 16 * h + 16; e += 8) {  // level * sc is exact
-        const uint32_t w = cw[e >> 3];
-        const f32x2 l0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0), l1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1);
-        const f32x2 l2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 2), l3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 3);
-        x[e] -= l0[0] * sc, x[e + 1] -= l0[1] * sc, x[e + 2] -= l1[0] * sc, x[e + 3] -= l1[1] * sc;
-        x[e + 4] -= l2[0] * sc, x[e + 5] -= l2[1] * sc, x[e + 6] -= l3[0] * sc, x[e + 7] -= l3[1] * sc;
+        float l[8];
+        fp4_levels8(cw[e >> 3], l);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[e + i] -= l[i] * sc;
       }
     }
     if (live) *(uint16_t *)((uint8_t *)s_pages + (blk * 64 + t) * 8 + 2 * g) = (uint16_t)sbs;
@@ -430,6 +544,8 @@ static int launch_status() {
   const hipError_t e = hipGetLastError();
   return e != hipSuccess ? ffa_set_error_internal(FFA_E_LAUNCH, hipGetErrorString(e)) : FFA_OK;
 }
+
+static bool aligned(const void *p, size_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
 
 static bool is_fp8(int dt) { return dt == FFA_DT_FP8_E4M3 || dt == FFA_DT_FP8_E5M2; }
 static bool is_float(int dt) { return dt >= FFA_DT_F16 && dt <= FFA_DT_F32; }
@@ -462,6 +578,21 @@ extern "C" int ffa_nvfp4_quantize(const void *k, int k_dtype, int B, int T, int 
   if (!is_float(k_dtype)) return ffa_set_error_internal(FFA_E_INVALID, "k dtype");
   if (!is_fp8(res_dtype)) return ffa_set_error_internal(FFA_E_INVALID, "residual dtype must be fp8");
   const int npg = (T + page_size - 1) / page_size;
+  if (D % 8 == 0 && aligned(k, 16) && aligned(residual, 8) && aligned(k_packed, 4)) {
+    const bool e4m3 = res_dtype == FFA_DT_FP8_E4M3;
+#define FFA_CASE(KK, EE)                                                                                              \
+  if (k_dtype == KK && e4m3 == EE)                                                                                    \
+    hipLaunchKernelGGL((ffa::nvfp4_quant8_kernel<KK, EE>), dim3(HKV, npg, B), dim3(256), 0, (hipStream_t)stream, k, T, \
+                       HKV, D, page_size, k_packed, scale, residual);
+    FFA_CASE(FFA_DT_F16, true)
+    FFA_CASE(FFA_DT_F16, false)
+    FFA_CASE(FFA_DT_BF16, true)
+    FFA_CASE(FFA_DT_BF16, false)
+    FFA_CASE(FFA_DT_F32, true)
+    FFA_CASE(FFA_DT_F32, false)
+#undef FFA_CASE
+    return launch_status();
+  }
   hipLaunchKernelGGL(ffa::nvfp4_quant_kernel, dim3(HKV, npg, B), dim3(256), 0, (hipStream_t)stream, k, k_dtype, T,
                      HKV, D, page_size, k_packed, scale, residual, res_dtype == FFA_DT_FP8_E4M3 ? 1 : 0);
   return launch_status();
@@ -489,8 +620,6 @@ extern "C" int ffa_nf4_quantize(const void *k, int k_dtype, int B, int T, int HK
                      HKV, D, (const float *)absmax, nsplit, k_packed, residual, res_dtype == FFA_DT_FP8_E4M3 ? 1 : 0);
   return launch_status();
 }
-
-static bool aligned(const void *p, size_t n) { return (reinterpret_cast<uintptr_t>(p) & (n - 1)) == 0; }
 
 static int group_append(bool nf4, const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
                         const int32_t *block_table, int bt_stride, int num_pages, uint8_t *k_pages,

@@ -276,3 +276,35 @@ def test_page_append_equals_token_append(gpu, fmt, k_dt, B, Tn, HKV, pos):
     for x, y in zip(wp, pp):
         assert np.array_equal(_u8(x), _u8(y))
     assert any((_u8(x) != 0x5A).any() for x in wp)
+
+
+# ------------------------------------------------------------------- nvfp4 / nf4 / fp8 in the reference layouts
+@pytest.mark.gpu
+@pytest.mark.parametrize("tau", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("B,T,HKV,D,page", [(1, 1, 1, 8, 128), (2, 130, 3, 24, 128), (1, 300, 2, 128, 64),
+                                            (1, 700, 2, 128, 512), (1, 77, 5, 64, 16), (2, 129, 8, 128, 128)])
+def test_nvfp4_quantizer_vector_route_equals_scalar_route(gpu, tau, B, T, HKV, D, page):
+    """Every byte of the vector kernel's route equals the scalar route's (keys at an odd address): pages held in
+    registers and read again, ragged last pages, keys on the codes' turning points, zeros, infinities, NaNs."""
+    from ffa_mi355x import kfmt_quant as KQ
+
+    dt = TORCH_DT[tau]
+    g = torch.Generator().manual_seed(T + page)
+    k = (torch.randn(B, T, HKV, D, generator=g) * 3).to(dt)
+    if T > 16:
+        k[0, :4, 0, :8] = 0.0
+        s = torch.tensor(3.7).to(dt)
+        k[:, 4] = k[:, 4].clamp(-1, 1) * s  # below the page's maximum
+        mids = torch.tensor([0.25, 0.75, 1.25, 1.75, 2.5, 3.5, 5.0])
+        k[0, 5, 0, :7], k[0, 6, 0, :7] = (mids * 2).to(dt), -(mids * 2).to(dt)
+        k[0, :page, HKV - 1] = k[0, :page, HKV - 1].clamp(-11, 11)
+        k[0, 7, HKV - 1, 0] = 12.0  # scale 2: the row of midpoints is exact
+        k[0, 5, HKV - 1, :7], k[0, 6, HKV - 1, :7] = (mids * 2).to(dt), -(mids * 2).to(dt)
+        k[-1, -1, 0, 1], k[-1, -1, 0, 2], k[-1, -2, 0, 3] = float("nan"), 1e-8, -1e-8
+        if B > 1:
+            k[0, 2, 1, 4] = float("inf")
+    k = k.to(gpu)
+    for fp8 in (torch.float8_e5m2, torch.float8_e4m3fn):
+        a, b = KQ.encode_nvfp4(k, fp8, page), KQ.encode_nvfp4(_misaligned(k), fp8, page)
+        for x, y in zip(a, b):
+            assert np.array_equal(_u8(x), _u8(y))
