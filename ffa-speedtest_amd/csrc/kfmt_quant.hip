@@ -348,7 +348,7 @@ __global__ __launch_bounds__(256) void kfmt_group_append_kernel(const void *k, i
                                                                  const int32_t *pos, const int32_t *bt, int bt_stride,
                                                                  int num_pages, uint8_t *k_pages, void *s_pages,
                                                                  uint8_t *r_pages, int res_e4m3, const void *v_new,
-                                                                 void *v_pages) {
+                                                                 int vmode, void *v_pages) {
   constexpr int D = 128;
   const size_t id = (size_t)blockIdx.x * 256 + threadIdx.x;
   const bool live = id < (size_t)M * HKV * 8;  // whole groups of 8 lanes are live or not
@@ -404,9 +404,9 @@ __global__ __launch_bounds__(256) void kfmt_group_append_kernel(const void *k, i
   *(uint2 *)(k_pages + blk * (64 * 64) + k4_off(slot, 8 * c16)) = make_uint2(cw[0], cw[1]);
   *(uint4 *)(r_pages + blk * (64 * D) + res_off(slot, 16 * c16)) = make_uint4(rw[0], rw[1], rw[2], rw[3]);
   if (v_new != nullptr) {
-    const uint16_t *vs = (const uint16_t *)v_new + ((size_t)m * HKV + hkv) * D + 16 * c16;
+    const size_t vs = ((size_t)m * HKV + hkv) * D + 16 * c16;
     uint16_t *vd = (uint16_t *)v_pages + blk * (D * 64);
-    for (int e = 0; e < 16; ++e) vd[vt_off(16 * c16 + e, slot)] = vs[e];
+    for (int e = 0; e < 16; ++e) vd[vt_off(16 * c16 + e, slot)] = v_element(v_new, vmode, vs + e);
   }
 }
 
@@ -623,8 +623,8 @@ extern "C" int ffa_nf4_quantize(const void *k, int k_dtype, int B, int T, int HK
 
 static int group_append(bool nf4, const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
                         const int32_t *block_table, int bt_stride, int num_pages, uint8_t *k_pages,
-                        void *scale_pages, uint8_t *res_pages, int res_dtype, const void *v_new, void *v_pages,
-                        void *stream) {
+                        void *scale_pages, uint8_t *res_pages, int res_dtype, const void *v_new, int vmode,
+                        void *v_pages, void *stream) {
   if (B <= 0 || Tn <= 0 || HKV <= 0) return ffa_set_error_internal(FFA_E_INVALID, "bad dims");
   if (bt_stride <= 0 || num_pages <= 0) return ffa_set_error_internal(FFA_E_INVALID, "empty block table or pool");
   if (!is_float(k_dtype)) return ffa_set_error_internal(FFA_E_INVALID, "k dtype");
@@ -640,7 +640,7 @@ static int group_append(bool nf4, const void *k, int k_dtype, int B, int Tn, int
   if (nf4 == NN && k_dtype == KK && e4m3 == EE)                                                                       \
     hipLaunchKernelGGL((ffa::kfmt_page_append_kernel<NN, KK, EE>), tiles, dim3(256), 0, (hipStream_t)stream, k, Tn,   \
                        HKV, pos, block_table, bt_stride, num_pages, k_pages, scale_pages, res_pages, v_new,           \
-                       ffa::kVSame, v_pages);
+                       vmode, v_pages);
 #define FFA_CASES(NN, KK) FFA_CASE(NN, KK, true) FFA_CASE(NN, KK, false)
     FFA_CASES(true, FFA_DT_F16)
     FFA_CASES(true, FFA_DT_BF16)
@@ -658,11 +658,11 @@ static int group_append(bool nf4, const void *k, int k_dtype, int B, int Tn, int
   if (nf4)
     hipLaunchKernelGGL(ffa::kfmt_group_append_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, k, k_dtype, B * Tn,
                        Tn, HKV, pos, block_table, bt_stride, num_pages, k_pages, scale_pages, res_pages, e4, v_new,
-                       v_pages);
+                       vmode, v_pages);
   else
     hipLaunchKernelGGL(ffa::kfmt_group_append_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, k, k_dtype,
                        B * Tn, Tn, HKV, pos, block_table, bt_stride, num_pages, k_pages, scale_pages, res_pages, e4,
-                       v_new, v_pages);
+                       v_new, vmode, v_pages);
   return launch_status();
 }
 
@@ -671,7 +671,7 @@ extern "C" int ffa_nvfp4_g16_append(const void *k, int k_dtype, int B, int Tn, i
                                     uint8_t *scale_pages, uint8_t *res_pages, int res_dtype, const void *v_new,
                                     void *v_pages, void *stream) {
   return group_append(false, k, k_dtype, B, Tn, HKV, pos, block_table, bt_stride, num_pages, k_pages, scale_pages,
-                      res_pages, res_dtype, v_new, v_pages, stream);
+                      res_pages, res_dtype, v_new, ffa::kVSame, v_pages, stream);
 }
 
 extern "C" int ffa_nf4_g64_append(const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
@@ -679,5 +679,25 @@ extern "C" int ffa_nf4_g64_append(const void *k, int k_dtype, int B, int Tn, int
                                   void *scale_pages, uint8_t *res_pages, int res_dtype, const void *v_new,
                                   void *v_pages, void *stream) {
   return group_append(true, k, k_dtype, B, Tn, HKV, pos, block_table, bt_stride, num_pages, k_pages, scale_pages,
-                      res_pages, res_dtype, v_new, v_pages, stream);
+                      res_pages, res_dtype, v_new, ffa::kVSame, v_pages, stream);
+}
+
+extern "C" int ffa_nvfp4_g16_append_cast(const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
+                                    const int32_t *block_table, int bt_stride, int num_pages, uint8_t *k_pages,
+                                    uint8_t *scale_pages, uint8_t *res_pages, int res_dtype, const void *v_new,
+                                    int v_new_dtype, void *v_pages, int v_dtype, void *stream) {
+  const int vmode = v_new ? ffa::v_mode(v_new_dtype, v_dtype) : ffa::kVSame;
+  if (vmode < 0) return ffa_set_error_internal(FFA_E_INVALID, "v dtypes (rows fp16, bf16 or fp32, pool fp16 or bf16)");
+  return group_append(false, k, k_dtype, B, Tn, HKV, pos, block_table, bt_stride, num_pages, k_pages, scale_pages,
+                      res_pages, res_dtype, v_new, vmode, v_pages, stream);
+}
+
+extern "C" int ffa_nf4_g64_append_cast(const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
+                                    const int32_t *block_table, int bt_stride, int num_pages, uint8_t *k_pages,
+                                    void *scale_pages, uint8_t *res_pages, int res_dtype, const void *v_new,
+                                    int v_new_dtype, void *v_pages, int v_dtype, void *stream) {
+  const int vmode = v_new ? ffa::v_mode(v_new_dtype, v_dtype) : ffa::kVSame;
+  if (vmode < 0) return ffa_set_error_internal(FFA_E_INVALID, "v dtypes (rows fp16, bf16 or fp32, pool fp16 or bf16)");
+  return group_append(true, k, k_dtype, B, Tn, HKV, pos, block_table, bt_stride, num_pages, k_pages, scale_pages,
+                      res_pages, res_dtype, v_new, vmode, v_pages, stream);
 }

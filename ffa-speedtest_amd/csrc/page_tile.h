@@ -14,8 +14,22 @@
 
 namespace ffa {
 
-// V rows given with an append: how they are brought to the pool's 16-bit type
+// V rows given with an append: how they are brought to the pool's 16-bit type (the conversions of a torch cast:
+// through fp32, round to nearest even).  Cast by the caller instead, 16K x 1024 bf16 values for an fp16 pool were
+// 67 MB more to move, a launch and an allocation.
 enum { kVSame = 0, kVBf16ToF16 = 1, kVF16ToBf16 = 2, kVF32ToF16 = 3, kVF32ToBf16 = 4 };
+// element types (0 = f16, 1 = bf16, 2 = f32) of the rows and of the pool; -1: not one of the above
+inline int v_mode(int from, int to) {
+  if (to != 0 && to != 1) return -1;
+  if (from == to) return kVSame;
+  if (from == 2) return to == 0 ? kVF32ToF16 : kVF32ToBf16;
+  return from == 1 ? kVBf16ToF16 : (from == 0 ? kVF16ToBf16 : -1);
+}
+__device__ __forceinline__ uint16_t v_element(const void *v, int vmode, size_t i) {
+  if (vmode == kVSame) return ((const uint16_t *)v)[i];
+  const float x = load_any(v, i, vmode == kVF16ToBf16 ? 0 : (vmode == kVBf16ToF16 ? 1 : 2));
+  return (uint16_t)(vmode == kVF16ToBf16 || vmode == kVF32ToBf16 ? f32_to_bf16_bits(x) : f32_to_f16_bits(x));
+}
 
 struct PageTile {
   int page;    // pool page, or -1: nothing to write

@@ -656,7 +656,7 @@ __global__ __launch_bounds__(256) void q2_g32_append_kernel(const void *k, int k
                                                              const int32_t *pos, const int32_t *bt, int bt_stride,
                                                              int num_pages, uint8_t *kq_pages, uint16_t *s_pages,
                                                              uint16_t *z_pages, uint8_t *r_pages, int res_e4m3,
-                                                             const void *v_new, void *v_pages) {
+                                                             const void *v_new, int vmode, void *v_pages) {
   constexpr int D = 128;
   const size_t rowid = (size_t)blockIdx.x * 2 + (threadIdx.x >> 7);  // (token row, head)
   if (rowid >= (size_t)M * HKV) return;  // whole waves (a row is two waves)
@@ -670,7 +670,7 @@ __global__ __launch_bounds__(256) void q2_g32_append_kernel(const void *k, int k
   const float x = load_any(k, rowid * D + c, kdt);
   g32_quantize_lanes(x, page >= 0, page, slot, hkv, HKV, g, kq_pages, s_pages, z_pages, r_pages, res_e4m3);
   if (v_new != nullptr && page >= 0)
-    ((uint16_t *)v_pages)[((size_t)page * HKV + hkv) * (D * 64) + vt_off(c, slot)] = ((const uint16_t *)v_new)[rowid * D + c];
+    ((uint16_t *)v_pages)[((size_t)page * HKV + hkv) * (D * 64) + vt_off(c, slot)] = v_element(v_new, vmode, rowid * D + c);
 }
 
 
@@ -1044,10 +1044,10 @@ extern "C" int ffa_kproj_rope_q2_append(const void *h, const void *w_k, const vo
   return FFA_OK;
 }
 
-extern "C" int ffa_q2_quantize_g32_append(const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
-                                          const int32_t *block_table, int bt_stride, int num_pages,
-                                          uint8_t *k_q_pages, void *scale_pages, void *zero_pages, uint8_t *res_pages,
-                                          int res_dtype, const void *v_new, void *v_pages, void *stream) {
+static int q2_g32_append(const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
+                         const int32_t *block_table, int bt_stride, int num_pages, uint8_t *k_q_pages,
+                         void *scale_pages, void *zero_pages, uint8_t *res_pages, int res_dtype, const void *v_new,
+                         int vmode, void *v_pages, void *stream) {
   if (B <= 0 || Tn <= 0 || HKV <= 0) return ffa_set_error_internal(FFA_E_INVALID, "bad dims");
   if (bt_stride <= 0 || num_pages <= 0) return ffa_set_error_internal(FFA_E_INVALID, "empty block table or pool");
   if (!(k_dtype >= FFA_DT_F16 && k_dtype <= FFA_DT_F32)) return ffa_set_error_internal(FFA_E_INVALID, "k dtype");
@@ -1064,7 +1064,7 @@ extern "C" int ffa_q2_quantize_g32_append(const void *k, int k_dtype, int B, int
   if (k_dtype == KK && e4m3 == EE)                                                                                  \
     hipLaunchKernelGGL((ffa::q2_g32_page_kernel<KK, EE>), grid, dim3(256), 0, (hipStream_t)stream, k, Tn, HKV, pos, \
                        block_table, bt_stride, num_pages, k_q_pages, (uint16_t *)scale_pages, (uint16_t *)zero_pages, \
-                       res_pages, v_new, ffa::kVSame, v_pages);
+                       res_pages, v_new, vmode, v_pages);
     FFA_CASE(FFA_DT_F16, true)
     FFA_CASE(FFA_DT_F16, false)
     FFA_CASE(FFA_DT_BF16, true)
@@ -1077,11 +1077,30 @@ extern "C" int ffa_q2_quantize_g32_append(const void *k, int k_dtype, int B, int
     hipLaunchKernelGGL(ffa::q2_g32_append_kernel, dim3((unsigned)((rows + 1) / 2)), dim3(256), 0,
                        (hipStream_t)stream, k, k_dtype, B * Tn, Tn, HKV, pos, block_table, bt_stride, num_pages,
                        k_q_pages, (uint16_t *)scale_pages, (uint16_t *)zero_pages, res_pages, e4m3 ? 1 : 0, v_new,
-                       v_pages);
+                       vmode, v_pages);
   }
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return ffa_set_error_internal(FFA_E_LAUNCH, hipGetErrorString(e));
   return FFA_OK;
+}
+
+extern "C" int ffa_q2_quantize_g32_append(const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
+                                          const int32_t *block_table, int bt_stride, int num_pages,
+                                          uint8_t *k_q_pages, void *scale_pages, void *zero_pages, uint8_t *res_pages,
+                                          int res_dtype, const void *v_new, void *v_pages, void *stream) {
+  return q2_g32_append(k, k_dtype, B, Tn, HKV, pos, block_table, bt_stride, num_pages, k_q_pages, scale_pages,
+                       zero_pages, res_pages, res_dtype, v_new, ffa::kVSame, v_pages, stream);
+}
+
+extern "C" int ffa_q2_quantize_g32_append_cast(const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
+                                               const int32_t *block_table, int bt_stride, int num_pages,
+                                               uint8_t *k_q_pages, void *scale_pages, void *zero_pages,
+                                               uint8_t *res_pages, int res_dtype, const void *v_new, int v_new_dtype,
+                                               void *v_pages, int v_dtype, void *stream) {
+  const int vmode = v_new ? ffa::v_mode(v_new_dtype, v_dtype) : ffa::kVSame;
+  if (vmode < 0) return ffa_set_error_internal(FFA_E_INVALID, "v dtypes (rows fp16, bf16 or fp32, pool fp16 or bf16)");
+  return q2_g32_append(k, k_dtype, B, Tn, HKV, pos, block_table, bt_stride, num_pages, k_q_pages, scale_pages,
+                       zero_pages, res_pages, res_dtype, v_new, vmode, v_pages, stream);
 }
 
 extern "C" int ffa_q2_paged_dequant(const uint8_t *k_q_pages, const void *scale_pages, const void *zero_pages,

@@ -36,6 +36,7 @@ EXPORTS = (
     "ffa_kproj_rope_q2_channel",
     "ffa_kproj_rope_q2_append",
     "ffa_q2_quantize_g32_append",
+    "ffa_q2_quantize_g32_append_cast",
     "ffa_q2_paged_dequant",
     "ffa_kproj_rope",
     "ffa_fp8fp8_quantize",
@@ -45,6 +46,8 @@ EXPORTS = (
     "ffa_nf4_quantize",
     "ffa_nvfp4_g16_append",
     "ffa_nf4_g64_append",
+    "ffa_nvfp4_g16_append_cast",
+    "ffa_nf4_g64_append_cast",
     "ffa_last_error",
     "ffa_version",
 )
@@ -201,6 +204,9 @@ def lib() -> ctypes.CDLL:
         L.ffa_kproj_rope_q2_append.restype = ci
         L.ffa_q2_quantize_g32_append.argtypes = [vp, ci, ci, ci, ci, vp, vp, ci, ci, vp, vp, vp, vp, ci, vp, vp, vp]
         L.ffa_q2_quantize_g32_append.restype = ci
+        L.ffa_q2_quantize_g32_append_cast.argtypes = [vp, ci, ci, ci, ci, vp, vp, ci, ci, vp, vp, vp, vp, ci, vp, ci,
+                                                      vp, ci, vp]
+        L.ffa_q2_quantize_g32_append_cast.restype = ci
         L.ffa_q2_paged_dequant.argtypes = [vp, vp, vp, vp, ci, vp, ci, vp, ci, ci, vp, ci, ci, ci, vp, vp, ci, vp]
         L.ffa_q2_paged_dequant.restype = ci
         L.ffa_kproj_rope.argtypes = [vp, vp, vp, ci, vp, vp, ci, ci, ci, ci, ci, ci, vp, vp]
@@ -217,6 +223,9 @@ def lib() -> ctypes.CDLL:
         L.ffa_nf4_quantize.restype = ci
         for name in ("ffa_nvfp4_g16_append", "ffa_nf4_g64_append"):
             getattr(L, name).argtypes = [vp, ci, ci, ci, ci, vp, vp, ci, ci, vp, vp, vp, ci, vp, vp, vp]
+            getattr(L, name).restype = ci
+        for name in ("ffa_nvfp4_g16_append_cast", "ffa_nf4_g64_append_cast"):
+            getattr(L, name).argtypes = [vp, ci, ci, ci, ci, vp, vp, ci, ci, vp, vp, vp, ci, vp, ci, vp, ci, vp]
             getattr(L, name).restype = ci
         _lib = L
         return _lib

@@ -74,6 +74,13 @@ def scale_pos(t):
     return 16 * (t // 16) + 4 * (t % 4) + (t // 4) % 4
 
 
+def append_rows(v: torch.Tensor, v_dtype: torch.dtype) -> torch.Tensor:
+    """V rows as the append kernels take them: contiguous, of a type that they bring to the pool's themselves."""
+    if v.dtype not in (torch.float16, torch.bfloat16, torch.float32):
+        v = v.to(v_dtype)
+    return v.contiguous()
+
+
 def check_append_fits(pos: torch.Tensor, Tn: int, block_table: torch.Tensor, num_pages: int) -> None:
     """Host-side bounds check of an append (positions and page ids must stay inside the table / pool)."""
     if block_table.shape[0] != pos.shape[0]:
@@ -108,19 +115,21 @@ class PagedQ2Cache:
         if HKV != self.HKV or D != HEAD_DIM:
             raise ValueError("k shape does not match the cache")
         k = k.contiguous()
+        v_from = v_to = N.DT_F16
         if v is not None:
             if v.shape != k.shape:
                 raise ValueError("v must have the shape of k")
-            v = v.to(self.v_dtype).contiguous()
+            v = append_rows(v, self.v_dtype)
+            v_from, v_to = N.dtype_code(v.dtype), N.dtype_code(self.v_dtype)
         pos = pos.to(torch.int32).contiguous()
         block_table = block_table.to(torch.int32).contiguous()
         check_append_fits(pos, Tn, block_table, self.P)
-        rc = N.lib().ffa_q2_quantize_g32_append(
+        rc = N.lib().ffa_q2_quantize_g32_append_cast(
             k.data_ptr(), N.dtype_code(k.dtype), B, Tn, HKV, pos.data_ptr(), block_table.data_ptr(),
             block_table.shape[1], self.P, self.k_q.data_ptr(), self.k_scale.data_ptr(), self.k_zero.data_ptr(),
-            self.k_res.data_ptr(), N.dtype_code(self.res_dtype), N.ptr(v), self.v.data_ptr(),
+            self.k_res.data_ptr(), N.dtype_code(self.res_dtype), N.ptr(v), v_from, self.v.data_ptr(), v_to,
             N.stream_of(k.device))
-        N.check(rc, "ffa_q2_quantize_g32_append")
+        N.check(rc, "ffa_q2_quantize_g32_append_cast")
 
     def dequantize(self, block_table: torch.Tensor, T: int, seq_lens: torch.Tensor | None = None,
                    out_dtype: torch.dtype = torch.float32):

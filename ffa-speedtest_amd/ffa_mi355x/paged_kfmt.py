@@ -24,7 +24,7 @@ import torch
 from . import _native as N
 from .decode import HEAD_DIM, DecodeWorkspace
 from .kfmt import run_kfmt_decode
-from .paged import PAGE, check_append_fits
+from .paged import PAGE, append_rows, check_append_fits
 
 FORMATS = ("nvfp4", "nf4")
 
@@ -107,17 +107,19 @@ class PagedKfmtCache:
         if HKV != self.HKV or D != HEAD_DIM:
             raise ValueError("k shape does not match the cache")
         k = k.contiguous()
+        v_from = v_to = N.DT_F16
         if v is not None:
             if v.shape != k.shape:
                 raise ValueError("v must have the shape of k")
-            v = v.to(self.v_dtype).contiguous()
+            v = append_rows(v, self.v_dtype)
+            v_from, v_to = N.dtype_code(v.dtype), N.dtype_code(self.v_dtype)
         pos = pos.to(device=k.device, dtype=torch.int32).contiguous()
         block_table = block_table.to(device=k.device, dtype=torch.int32).contiguous()
         check_append_fits(pos, Tn, block_table, self.P)
-        fn = N.lib().ffa_nvfp4_g16_append if self.fmt == "nvfp4" else N.lib().ffa_nf4_g64_append
+        fn = N.lib().ffa_nvfp4_g16_append_cast if self.fmt == "nvfp4" else N.lib().ffa_nf4_g64_append_cast
         rc = fn(k.data_ptr(), N.dtype_code(k.dtype), B, Tn, HKV, pos.data_ptr(), block_table.data_ptr(),
                 block_table.shape[1], self.P, self.k.data_ptr(), self.k_scale.data_ptr(), self.k_res.data_ptr(),
-                N.dtype_code(self.res_dtype), N.ptr(v), self.v.data_ptr(), N.stream_of(k.device))
+                N.dtype_code(self.res_dtype), N.ptr(v), v_from, self.v.data_ptr(), v_to, N.stream_of(k.device))
         N.check(rc, f"ffa_{self.fmt}_append")
 
     def decode(self, q, block_table, seq_lens=None, **kw) -> DecodeWorkspace:

@@ -29,6 +29,9 @@
  *                             reference-layout cache with its existing per-channel scale / zero
  *   ffa_q2_quantize_g32_append no reference counterpart: g32 quantize + paged append of
  *                             given K rows (the paged g32 cache layout)
+ *   ffa_q2_quantize_g32_append_cast, the paged appends with V rows of another type than the pool's
+ *   ffa_nvfp4_g16_append_cast,
+ *   ffa_nf4_g64_append_cast
  *   ffa_q2_paged_dequant      ffa-fp8fp8/e2e/fp8fp8_cache.py:60-69, 84-89 (_refresh_fp_cache:
  *                             the cache's keys dequantized for exact attention), for the
  *                             paged g32 cache
@@ -282,6 +285,16 @@ int ffa_q2_quantize_g32_append(const void *k, int k_dtype, int B, int Tn, int HK
                                const void *v_new, void *v_pages, void *stream);
 
 /*
+ * The same with the V rows in another type than the pool's: v_new [B, Tn, HKV, 128] of v_new_dtype
+ * (F16/BF16/F32), written to a pool of v_dtype (F16/BF16) as a cast rounds it (through fp32, to
+ * nearest even).
+ */
+int ffa_q2_quantize_g32_append_cast(const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
+                                    const int32_t *block_table, int bt_stride, int num_pages, uint8_t *k_q_pages,
+                                    void *scale_pages, void *zero_pages, uint8_t *res_pages, int res_dtype,
+                                    const void *v_new, int v_new_dtype, void *v_pages, int v_dtype, void *stream);
+
+/*
  * Paged g32 cache -> contiguous K and V [B, T, HKV, 128] in out_dtype (F16/BF16/F32), the keys
  * dequantized as k = c * scale + zero + residual (fp32, one rounding to out_dtype) and V copied
  * from the V^T pages (v_dtype F16/BF16).  T is a multiple of 64; tokens at or past seq_lens[b]
@@ -341,6 +354,15 @@ int ffa_nvfp4_g16_append(const void *k, int k_dtype, int B, int Tn, int HKV, con
 int ffa_nf4_g64_append(const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
                        const int32_t *block_table, int bt_stride, int num_pages, uint8_t *k_pages, void *scale_pages,
                        uint8_t *res_pages, int res_dtype, const void *v_new, void *v_pages, void *stream);
+/* The two with V rows of v_new_dtype for a pool of v_dtype, as ffa_q2_quantize_g32_append_cast. */
+int ffa_nvfp4_g16_append_cast(const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
+                              const int32_t *block_table, int bt_stride, int num_pages, uint8_t *k_pages,
+                              uint8_t *scale_pages, uint8_t *res_pages, int res_dtype, const void *v_new,
+                              int v_new_dtype, void *v_pages, int v_dtype, void *stream);
+int ffa_nf4_g64_append_cast(const void *k, int k_dtype, int B, int Tn, int HKV, const int32_t *pos,
+                            const int32_t *block_table, int bt_stride, int num_pages, uint8_t *k_pages,
+                            void *scale_pages, uint8_t *res_pages, int res_dtype, const void *v_new, int v_new_dtype,
+                            void *v_pages, int v_dtype, void *stream);
 int ffa_nf4_quantize(const void *k, int k_dtype, int B, int T, int HKV, int D, uint8_t *k_packed, void *scale,
                      uint8_t *residual, int res_dtype, float *absmax, void *stream);
 
