@@ -314,3 +314,26 @@ def test_nvfp4_quantizer_vector_route_equals_scalar_route(gpu, tau, B, T, HKV, D
         a, b = KQ.encode_nvfp4(k, fp8, page), KQ.encode_nvfp4(_misaligned(k), fp8, page)
         for x, y in zip(a, b):
             assert np.array_equal(_u8(x), _u8(y))
+
+
+@pytest.mark.parametrize("limit", [16384, 0])
+@pytest.mark.parametrize("pos,Tn,table,pages,error", [
+    ([0, 70], 58, [[3, 1], [0, 2]], 4, None),
+    ([0, 70], 59, [[3, 1], [0, 2]], 4, "positions exceed"),
+    ([-1, 0], 1, [[3, 1], [0, 2]], 4, "positions exceed"),
+    ([0, 1], 5, [[3, -1], [0, 9]], 4, None),   # the second column is not reached
+    ([0, 60], 5, [[3, -1], [0, 2]], 4, "outside the pool"),
+    ([0, 60], 5, [[3, 1], [0, 4]], 4, "outside the pool"),
+    ([0], 1, [[0], [1]], 4, "one row per sequence"),
+])
+def test_append_bounds_check(monkeypatch, limit, pos, Tn, table, pages, error):
+    """The append's bounds check, with the table read whole or reduced where it lies."""
+    from ffa_mi355x import paged
+
+    monkeypatch.setattr(paged, "_CHECK_ON_HOST", limit)
+    args = torch.tensor(pos, dtype=torch.int32), Tn, torch.tensor(table, dtype=torch.int32), pages
+    if error is None:
+        paged.check_append_fits(*args)
+    else:
+        with pytest.raises(ValueError, match=error):
+            paged.check_append_fits(*args)
