@@ -128,9 +128,10 @@ void kfmt_decode_kernel(const DecodeParams p) {
   // the paged small-grid builds place the KV head fastest instead, so that a (sequence, KV head)'s
   // partials stay in one XCD's L2 for the merge (grid_pos).  In the paged large-batch build the KV
   // head fastest took config 4 from 139.8 to 141.7 us (config 3 86.6 -> 86.1 us)
-  const GridPos gp = grid_pos<(LAYOUT == kContig && !k4) || (LAYOUT == kPaged && !RELOAD)>();
+  constexpr bool kUnitFastest = (LAYOUT == kContig && !k4) || (LAYOUT == kPaged && !RELOAD);
+  const GridPos gp = grid_pos<kUnitFastest>();
   const int cg = gp.cg;  // workgroup index along the sequence = partial slot
-  const DecodeUnit un = decode_unit(p, gp.y);  // KV head and the (at most 4) query rows of this workgroup
+  const DecodeUnit un = decode_unit<kUnitFastest>(p, gp.y);  // KV head and the (at most 4) query rows of this workgroup
   const int hkv = un.hkv;
   const int b = gp.b;
   // span: chunks of this workgroup (8, or 4 / 2 for small grids, where each wave owns one chunk
@@ -189,7 +190,8 @@ void kfmt_decode_kernel(const DecodeParams p) {
   const int NTBS_b = NTB * div_pow2(p.BS, p.SBS);
   const int NTBk = div_bs(p, p.T + p.BS - 1);  // blocks of the block-scale tensor
   // probe windows: waves 0 and 1 (SPEC: 2 and 3, the waves with the operands)
-  const bool do_probe = (p.th_in == nullptr) && wch < 2;
+  // (pass 2 has pass 1's decisions)
+  const bool do_probe = (p.th_in == nullptr) && wch < 2 && p.pass != 2;
   const int pa = wch == 0 ? 0 : max(NTB - 1, 0) * 16;  // probe window (attn_kernel...q2fp8.py:58-73)
   int nv[kPPW];  // valid tokens of the wave's chunks (0 for a chunk it does not own)
 #pragma unroll

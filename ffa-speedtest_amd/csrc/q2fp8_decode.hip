@@ -143,7 +143,11 @@ __host__ __device__ constexpr int scale_pos(int t) { return 16 * (t >> 4) + 4 * 
 // waves 0 and 1, which would own none, load the residual and V rows of chunk wv (the chunk of wave
 // wv + 2) right after the operand barrier, before the prune decides it, and refine that chunk from
 // their registers if it is kept.
-template <int LAYOUT, int SMODE, int RES, int VT, int OCC, bool SPEC>
+// SHARE (paged g32 with several quads of query rows per KV head): the quads' workgroups read the same codes,
+// scales, residual and V from one XCD's L2 (decode_unit), so these loads keep the default cache policy
+// (bload16_nt's, for data that one workgroup reads: 68.5 against 62.8 us for 8 sequences of 3K-16K tokens with 64
+// query heads; one quad without the hint, 32K tokens, 16 layers: 219 against 204 us).
+template <int LAYOUT, int SMODE, int RES, int VT, int OCC, bool SPEC, bool SHARE>
 __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
   static_assert(!SPEC || (OCC == 1 && (LAYOUT == kPaged) == (SMODE == kG32)),
                 "the two-chunk builds: paged g32, contiguous per-channel");
@@ -161,7 +165,7 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
   // the merge (grid_pos)
   const GridPos gp = grid_pos<LAYOUT == kPaged>();
   const int cg = gp.cg;  // workgroup index along the sequence = partial slot
-  const DecodeUnit un = decode_unit(p, gp.y);  // KV head and the (at most 4) query rows of this workgroup
+  const DecodeUnit un = decode_unit<LAYOUT == kPaged>(p, gp.y);  // KV head and the (at most 4) query rows of this workgroup
   const int hkv = un.hkv;
   const int b = gp.b;
   // span: chunks of this workgroup (8, or 4 / 2 for small grids, where each wave owns one chunk and
@@ -213,6 +217,10 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
   float(*const s_zs)[64] = reinterpret_cast<float(*)[64]>(&s_po[2][0][0]);
   __shared__ __attribute__((aligned(16))) uint8_t s_vstage[LAYOUT == kContig ? kWaves * kPage * kVRowHalf : 16];
 
+  auto load16 = [](brsrc r, uint32_t off) {
+    if constexpr (SHARE) return bload16(r, off);
+    else return bload16_nt(r, off);
+  };
   // Workgroup barrier for LDS traffic only: __syncthreads() would also wait for every
   // outstanding global load of the wave (s_waitcnt vmcnt(0)), serialising the page loads
   // issued ahead of it.
@@ -235,11 +243,40 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
   const int NTB = div_bs(p, Tb + p.BS - 1);
   const int NTBS_b = NTB * div_pow2(p.BS, p.SBS);
   // probe windows: waves 0 and 1 (SPEC: 2 and 3, which score)
-  const bool do_probe = (p.th_in == nullptr) && wch < 2;
+  // (pass 2 has pass 1's decisions)
+  const bool do_probe = (p.th_in == nullptr) && wch < 2 && p.pass != 2;
   const int pa = wch == 0 ? 0 : max(NTB - 1, 0) * 16;  // probe window (attn_kernel...q2fp8.py:58-73)
   int nv[kPPW];  // valid tokens of the wave's chunks (0 for a chunk it does not own)
 #pragma unroll
   for (int j = 0; j < kPPW; ++j) nv[j] = own[j] ? min(max(Tb - (c0 + j) * kPage, 0), kPage) : 0;
+  // Two-pass decodes with many workgroups decide before they load: pass 1 has every block's maxima, so a pruned
+  // chunk's codes need not be read and scored again, and a workgroup without a kept block writes its empty
+  // partial and is done (4 sequences of 64K tokens, 64 query heads, 12 % kept: 119 -> 106 us; 8 of 3K-16K, 57 %
+  // kept: 63.3 -> 64).  The mean-V fallback needs the pruned tokens' scores.
+  const bool early = SHARE && OCC > 1 && p.pass == 2 && p.v_mean == nullptr;
+  if (early) {
+    lds_barrier();  // s_keep is zero
+    decide_blocks(p, b, hkv, cw, Tb, s_keep);
+    lds_barrier();
+    const int nblk = SBS <= kChunksPerWG * kPage ? div_pow2(kChunksPerWG * kPage, SBS) : 1;
+    const uint32_t kb = (uint32_t)__ballot(lane < nblk && s_keep[lane < nblk ? lane : 0] != 0);  // at most 32 blocks
+    if (kb == 0u) {
+      if (un.quad == 0) write_empty_mask(p.mask + ((size_t)b * p.HKV + hkv) * p.ntbs, cg, SBS, p.ntbs, span);
+      if (threadIdx.x < un.Gu) {
+        const size_t row = (size_t)b * p.HQ + un.row0 + threadIdx.x;
+        p.m_buf[row * p.nparts + cg] = -INFINITY;
+        p.l_buf[row * p.nparts + cg] = 0.f;
+      }
+      return;
+    }
+#pragma unroll
+    for (int j = 0; j < kPPW; ++j) {
+      const int c = wch * ppw + j;  // chunk within the span
+      const int per = SBS <= kPage ? div_pow2(kPage, SBS) : 1;  // its blocks
+      const uint32_t bits = ((1u << per) - 1u) << (SBS <= kPage ? c * per : (nblk > 1 ? div_pow2(c * kPage, SBS) : 0));
+      if ((kb & bits) == 0u) nv[j] = 0;
+    }
+  }
   // SPEC: the chunk whose residual and V^T waves 0 and 1 load (chunk wv), and its valid tokens
   const int lc = cw + (wv & 1);
   const int nl = SPEC && wv < 2 ? min(max(Tb - lc * kPage, 0), kPage) : 0;
@@ -311,7 +348,7 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
       const size_t blk = (size_t)pg[j] * p.HKV + hkv;
       const brsrc rc = make_rsrc(p.kq + blk * (4 * kPage * 8), nv[j] > 0 ? 4 * kPage * 8 : 0);
       // tokens 4 mrow + (0, 1) and 4 mrow + (2, 3) of group kc: two 1 KB blocks, lane-ordered
-      const uint4 q0 = bload16_nt(rc, lane * 16), q1 = bload16_nt(rc, (64 + lane) * 16);
+      const uint4 q0 = load16(rc, lane * 16), q1 = load16(rc, (64 + lane) * 16);
       x[j][0] = ((uint64_t)q0.y << 32) | q0.x;
       x[j][1] = ((uint64_t)q0.w << 32) | q0.z;
       x[j][2] = ((uint64_t)q1.y << 32) | q1.x;
@@ -321,10 +358,10 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
         const brsrc rz = make_rsrc((const uint16_t *)p.kz + blk * (4 * kPage), nv[j] > 0 ? 4 * kPage * 2 : 0);
         // slots 16 kc + (0..7) and 16 kc + (8..15) of group jg
         const uint32_t so0 = gscale_off(jg, 16 * kc) * 2, so1 = gscale_off(jg, 16 * kc + 8) * 2;
-        gs[j][0] = bload16_nt(rs, so0);
-        gs[j][1] = bload16_nt(rs, so1);
-        gz[j][0] = bload16_nt(rz, so0);
-        gz[j][1] = bload16_nt(rz, so1);
+        gs[j][0] = load16(rs, so0);
+        gs[j][1] = load16(rs, so1);
+        gz[j][0] = load16(rz, so0);
+        gz[j][1] = load16(rz, so1);
       }
     } else {
       const size_t base = (((size_t)b * p.T + t0) * p.HKV + hkv) * 32;
@@ -426,15 +463,15 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
         const brsrc rs = make_rsrc(p.kr + blk * (kPage * kD), nl > 0 ? kPage * kD : 0);
 #pragma unroll
         for (int tau = 0; tau < 4; ++tau) {
-          srr[tau][0] = bload16_nt(rs, ((tau * 2 + 0) * 64 + lane) * 16);
-          srr[tau][1] = bload16_nt(rs, ((tau * 2 + 1) * 64 + lane) * 16);
+          srr[tau][0] = load16(rs, ((tau * 2 + 0) * 64 + lane) * 16);
+          srr[tau][1] = load16(rs, ((tau * 2 + 1) * 64 + lane) * 16);
         }
       }
       const brsrc vs = make_rsrc((const uint16_t *)p.v + blk * (kD * kPage), nl > 0 ? kD * kPage * 2 : 0);
 #pragma unroll
       for (int nu = 0; nu < 8; ++nu)
 #pragma unroll
-        for (int kap = 0; kap < 2; ++kap) svv[nu][kap] = bload16_nt(vs, ((nu * 2 + kap) * 64 + lane) * 16);
+        for (int kap = 0; kap < 2; ++kap) svv[nu][kap] = load16(vs, ((nu * 2 + kap) * 64 + lane) * 16);
     }
   } else if constexpr (SPEC) {  // contiguous rows of tokens lc * 64 .. (the exact pass's load pattern)
     if (wv < 2) {
@@ -444,8 +481,8 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
 #pragma unroll
         for (int tau = 0; tau < 4; ++tau) {
           const uint32_t ro = (4 * mrow + tau) * p.HKV * kD + 32 * kc;
-          srr[tau][0] = bload16_nt(rs, ro);
-          srr[tau][1] = bload16_nt(rs, ro + 16);
+          srr[tau][0] = load16(rs, ro);
+          srr[tau][1] = load16(rs, ro + 16);
         }
       }
       const brsrc vs = make_rsrc((const uint16_t *)p.v + row0 * kD, nl > 0 ? ((nl - 1) * p.HKV + 1) * kD * 2 : 0);
@@ -453,7 +490,7 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
       for (int r = 0; r < 16; ++r) {
         const int idx = r * 64 + lane;
         const int tk = idx >> 4, vc = idx & 15;
-        svv[r >> 1][r & 1] = bload16_nt(vs, tk * p.HKV * kD * 2 + 16 * vc);
+        svv[r >> 1][r & 1] = load16(vs, tk * p.HKV * kD * 2 + 16 * vc);
       }
     }
   }
@@ -615,7 +652,7 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
     if (p.th_out != nullptr && cg == 0 && threadIdx.x < un.Gu) p.th_out[(size_t)b * p.HQ + un.row0 + threadIdx.x] = th;
     return;
   }
-  if (p.pass == 2) {  // second pass: decide from every row's maxima
+  if (p.pass == 2 && !early) {  // second pass: decide from every row's maxima
     decide_blocks(p, b, hkv, cw, Tb, s_keep);
     lds_barrier();
   }
@@ -764,11 +801,11 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
 #pragma unroll
       for (int tau = 0; tau < 4; ++tau) {
         if constexpr (LAYOUT == kPaged) {  // token 4 mrow + tau, channels 32 kc + 16 h + (0..15): block (tau, h)
-          rr[tau][0] = bload16_nt(rr_s, ((tau * 2 + 0) * 64 + lane) * 16);
-          rr[tau][1] = bload16_nt(rr_s, ((tau * 2 + 1) * 64 + lane) * 16);
+          rr[tau][0] = load16(rr_s, ((tau * 2 + 0) * 64 + lane) * 16);
+          rr[tau][1] = load16(rr_s, ((tau * 2 + 1) * 64 + lane) * 16);
         } else {
-          rr[tau][0] = bload16_nt(rr_s, ro[tau]);
-          rr[tau][1] = bload16_nt(rr_s, ro[tau] + 16);
+          rr[tau][0] = load16(rr_s, ro[tau]);
+          rr[tau][1] = load16(rr_s, ro[tau] + 16);
         }
       }
     }
@@ -777,7 +814,7 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
 #pragma unroll
       for (int nu = 0; nu < VH; ++nu)
 #pragma unroll
-        for (int kap = 0; kap < 2; ++kap) vv[nu][kap] = bload16_nt(vs_p, ((nu * 2 + kap) * 64 + lane) * 16);  // block (nu, kap)
+        for (int kap = 0; kap < 2; ++kap) vv[nu][kap] = load16(vs_p, ((nu * 2 + kap) * 64 + lane) * 16);  // block (nu, kap)
     } else {
       const brsrc vs = make_rsrc((const uint16_t *)p.v + (((size_t)b * p.T + t0) * p.HKV + hkv) * kD,
                                  ((nvs - 1) * p.HKV + 1) * kD * 2);
@@ -785,7 +822,7 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
       for (int r = 0; r < 16; ++r) {
         const int idx = r * 64 + lane;
         const int tk = idx >> 4, vc = idx & 15;
-        vv[r >> 1][r & 1] = bload16_nt(vs, tk * p.HKV * kD * 2 + 16 * vc);
+        vv[r >> 1][r & 1] = load16(vs, tk * p.HKV * kD * 2 + 16 * vc);
       }
     }
     }
@@ -888,7 +925,7 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
 #pragma unroll
             for (int n2 = VH; n2 < 8; ++n2)
 #pragma unroll
-              for (int kap = 0; kap < 2; ++kap) vv[n2][kap] = bload16_nt(vs_p, ((n2 * 2 + kap) * 64 + lane) * 16);
+              for (int kap = 0; kap < 2; ++kap) vv[n2][kap] = load16(vs_p, ((n2 * 2 + kap) * 64 + lane) * 16);
           }
 #pragma unroll
           for (int kap = 0; kap < 2; ++kap) {
@@ -1054,10 +1091,10 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
 #endif
 }
 
-template <int LAYOUT, int SMODE, int RES, int VT, int OCC>
+template <int LAYOUT, int SMODE, int RES, int VT, int OCC, bool SHARE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC))) void q2fp8_decode_kernel(
     const DecodeParams p) {
-  q2fp8_decode_body<LAYOUT, SMODE, RES, VT, OCC, false>(p);
+  q2fp8_decode_body<LAYOUT, SMODE, RES, VT, OCC, false, SHARE>(p);
 }
 
 // the decode of two-chunk spans (small grids of at most one workgroup per CU): paged g32 and the
@@ -1065,7 +1102,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OCC))) void
 template <int LAYOUT, int SMODE, int RES, int VT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void q2fp8_decode_2span_kernel(
     const DecodeParams p) {
-  q2fp8_decode_body<LAYOUT, SMODE, RES, VT, 1, true>(p);
+  q2fp8_decode_body<LAYOUT, SMODE, RES, VT, 1, true, false>(p);
 }
 
 // --------------------------------------------------------------------------
@@ -1347,8 +1384,16 @@ static hipError_t launch_decode(const ffa::DecodeParams &p, dim3 g0, hipStream_t
   // paged g32 with more workgroups than two per CU: the four-per-CU build of the kernel
   if constexpr (L == ffa::kPaged && S == ffa::kG32) {
     const int cus = ffa::device_cus();
-    if (cus > 0 && grid.x * grid.y * grid.z > 2u * (unsigned)cus) {
-      hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, 4>), grid, dim3(256), 0, st, p);
+    const bool many = cus > 0 && grid.x * grid.y * grid.z > 2u * (unsigned)cus;
+    if (p.nq > 1) {  // several quads of query rows per KV head share its data
+      if (many)
+        hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, 4, true>), grid, dim3(256), 0, st, p);
+      else
+        hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, 1, true>), grid, dim3(256), 0, st, p);
+      return hipGetLastError();
+    }
+    if (many) {
+      hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, 4, false>), grid, dim3(256), 0, st, p);
       return hipGetLastError();
     }
   }
@@ -1363,7 +1408,7 @@ static hipError_t launch_decode(const ffa::DecodeParams &p, dim3 g0, hipStream_t
   // fp32 channel scales: held to two workgroups per CU (the fp32 dequantization's temporaries would
   // otherwise take the kernel to 256 registers, one workgroup per CU)
   constexpr int occ = S == ffa::kChannelF32 ? 2 : 1;
-  hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, occ>), grid, dim3(256), 0, st, p);
+  hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, occ, false>), grid, dim3(256), 0, st, p);
   return hipGetLastError();
 }
 
