@@ -138,15 +138,17 @@ __host__ __device__ constexpr int scale_pos(int t) { return 16 * (t >> 4) + 4 * 
 // workgroups share a CU (29 KB of LDS each): used when the grid has more workgroups than two per
 // CU can hold (large batches), where it trades a few spilled registers for two more workgroups
 // in flight.
+// OCC = 3, contiguous per-channel: three workgroups per CU (168 registers, 52 KB of LDS with V staged a quarter of
+// its columns at a time and the channel scales kept once per channel group; OCC = 1: 230 registers, 69 KB, two).
 // SPEC (the builds for two-chunk spans, q2fp8_decode_2span_kernel: paged g32 and the contiguous
 // per-channel layouts): waves 2 and 3 own the two chunks and score them and the probe windows;
 // waves 0 and 1, which would own none, load the residual and V rows of chunk wv (the chunk of wave
 // wv + 2) right after the operand barrier, before the prune decides it, and refine that chunk from
 // their registers if it is kept.
-// SHARE (paged g32 with several quads of query rows per KV head): the quads' workgroups read the same codes,
-// scales, residual and V from one XCD's L2 (decode_unit), so these loads keep the default cache policy
-// (bload16_nt's, for data that one workgroup reads: 68.5 against 62.8 us for 8 sequences of 3K-16K tokens with 64
-// query heads; one quad without the hint, 32K tokens, 16 layers: 219 against 204 us).
+// SHARE (several quads of query rows per KV head; paged g32, contiguous per-channel): the quads' workgroups read the
+// same codes, scales, residual and V from the caches (paged: from one XCD's L2, decode_unit), so these loads keep
+// the default cache policy (bload16_nt's, for data that one workgroup reads: 68.5 against 62.8 us for 8 sequences
+// of 3K-16K tokens with 64 query heads; one quad without the hint, 32K tokens, 16 layers: 219 against 204 us).
 template <int LAYOUT, int SMODE, int RES, int VT, int OCC, bool SPEC, bool SHARE>
 __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
   static_assert(!SPEC || (OCC == 1 && (LAYOUT == kPaged) == (SMODE == kG32)),
@@ -191,9 +193,11 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
   const bool row_ok = ir < un.Gu;
   const int hq = un.row0 + (row_ok ? ir : 0);
 
-  __shared__ uint4 s_qr[4][64];                    // B operands of the 4 residual MFMAs (g32)
-  __shared__ uint4 s_sp[kG || kCF ? 1 : 4][kG || kCF ? 1 : 64];   // channel scales: fp16 (scale, scale) pairs of 8 channels
-  __shared__ uint4 s_zp2[kG || kCF ? 1 : 4][kG || kCF ? 1 : 64];  // channel scales: fp16 (zero, zero) pairs
+  __shared__ uint4 s_qr[kG ? 4 : 1][kG ? 64 : 1];  // B operands of the 4 residual MFMAs (g32)
+  // channel scales: fp16 (scale, scale) and (zero, zero) pairs of 8 channels of each channel group (the lanes of
+  // one group share them: broadcast reads)
+  __shared__ uint4 s_sp[kG || kCF ? 1 : 4][kG || kCF ? 1 : 4];
+  __shared__ uint4 s_zp2[kG || kCF ? 1 : 4][kG || kCF ? 1 : 4];
   // fp32 channel scales: [channel group kc][operand][s of elements 0-3, 4-7, z of 0-3, 4-7] (the
   // lanes of one kc share them: broadcast reads)
   __shared__ float4 s_cf[kCF ? 4 : 1][kCF ? 4 : 1][4];
@@ -215,7 +219,10 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
   uint4(*const s_qa)[64] = reinterpret_cast<uint4(*)[64]>(&s_po[0][0][0]);
   // g32: partial sums of q16 over 8 channels (read with the operands), after s_qa
   float(*const s_zs)[64] = reinterpret_cast<float(*)[64]>(&s_po[2][0][0]);
-  __shared__ __attribute__((aligned(16))) uint8_t s_vstage[LAYOUT == kContig ? kWaves * kPage * kVRowHalf : 16];
+  // contiguous V staging, per wave: half a tile's columns (64), in the many-workgroup build a quarter (32)
+  constexpr bool kBigC = LAYOUT == kContig && SMODE == kChannel && OCC > 1;
+  constexpr int kVCols = kBigC ? 32 : 64, kVPitch = kBigC ? 72 : kVRowHalf;
+  __shared__ __attribute__((aligned(16))) uint8_t s_vstage[LAYOUT == kContig ? kWaves * kPage * kVPitch : 16];
 
   auto load16 = [](brsrc r, uint32_t off) {
     if constexpr (SHARE) return bload16(r, off);
@@ -383,7 +390,7 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
     constexpr int s = w & 1;
     float qv[16];  // channels 32kc + 16h + (0..15)
     raw16_to_f32(qraw, p.q_dtype, qv);
-    u32x4 a4, r4;
+    u32x4 a4, r4 = {0, 0, 0, 0};
     if constexpr (kG) {
 #pragma unroll
       for (int qq = 0; qq < 4; ++qq) {
@@ -431,18 +438,22 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
           spw[qq] = f32_to_f16_bits(sv[8 * s + kChanPerm(2 * qq)]) | (f32_to_f16_bits(sv[8 * s + kChanPerm(2 * qq + 1)]) << 16);
           zpw[qq] = f32_to_f16_bits(zv[8 * s + kChanPerm(2 * qq)]) | (f32_to_f16_bits(zv[8 * s + kChanPerm(2 * qq + 1)]) << 16);
         }
-        s_sp[w][lane] = make_uint4(spw[0], spw[1], spw[2], spw[3]);
-        s_zp2[w][lane] = make_uint4(zpw[0], zpw[1], zpw[2], zpw[3]);
+        if (mrow == 0) {
+          s_sp[w][kc] = make_uint4(spw[0], spw[1], spw[2], spw[3]);
+          s_zp2[w][kc] = make_uint4(zpw[0], zpw[1], zpw[2], zpw[3]);
+        }
       }
     }
+    if constexpr (kG) {
 #pragma unroll
-    for (int qq = 0; qq < 4; ++qq) {
-      const float e0 = row_ok ? (float)(_Float16)qv[8 * s + 2 * qq] : 0.f;
-      const float e1 = row_ok ? (float)(_Float16)qv[8 * s + 2 * qq + 1] : 0.f;
-      r4[qq] = f32_to_f16_bits(e0) | (f32_to_f16_bits(e1) << 16);
+      for (int qq = 0; qq < 4; ++qq) {
+        const float e0 = row_ok ? (float)(_Float16)qv[8 * s + 2 * qq] : 0.f;
+        const float e1 = row_ok ? (float)(_Float16)qv[8 * s + 2 * qq + 1] : 0.f;
+        r4[qq] = f32_to_f16_bits(e0) | (f32_to_f16_bits(e1) << 16);
+      }
+      s_qr[w][lane] = make_uint4(r4[0], r4[1], r4[2], r4[3]);
     }
     s_qa[w][lane] = make_uint4(a4[0], a4[1], a4[2], a4[3]);
-    s_qr[w][lane] = make_uint4(r4[0], r4[1], r4[2], r4[3]);
   };
   switch (wv) {
     case 0: build_operands(std::integral_constant<int, 0>()); break;
@@ -502,7 +513,7 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
     const uint4 a = s_qa[mp][lane];
     qa[mp] = __builtin_bit_cast(f16x8, u32x4{a.x, a.y, a.z, a.w});
     if constexpr (!kG && !kCF) {
-      const uint4 sp = s_sp[mp][lane], zp = s_zp2[mp][lane];
+      const uint4 sp = s_sp[mp][kc], zp = s_zp2[mp][kc];
       spair[4 * mp + 0] = sp.x; spair[4 * mp + 1] = sp.y; spair[4 * mp + 2] = sp.z; spair[4 * mp + 3] = sp.w;
       zpair[4 * mp + 0] = zp.x; zpair[4 * mp + 1] = zp.y; zpair[4 * mp + 2] = zp.z; zpair[4 * mp + 3] = zp.w;
     }
@@ -816,13 +827,19 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
 #pragma unroll
         for (int kap = 0; kap < 2; ++kap) vv[nu][kap] = load16(vs_p, ((nu * 2 + kap) * 64 + lane) * 16);  // block (nu, kap)
     } else {
-      const brsrc vs = make_rsrc((const uint16_t *)p.v + (((size_t)b * p.T + t0) * p.HKV + hkv) * kD,
-                                 ((nvs - 1) * p.HKV + 1) * kD * 2);
+      vs_p = make_rsrc((const uint16_t *)p.v + (((size_t)b * p.T + t0) * p.HKV + hkv) * kD,
+                       ((nvs - 1) * p.HKV + 1) * kD * 2);
+      if constexpr (kBigC) {  // the first 64 columns: whole lines, 8 lanes a row
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int idx = r * 64 + lane;
-        const int tk = idx >> 4, vc = idx & 15;
-        vv[r >> 1][r & 1] = load16(vs, tk * p.HKV * kD * 2 + 16 * vc);
+        for (int r = 0; r < 8; ++r)
+          vv[r >> 1][r & 1] = load16(vs_p, (8 * r + (lane >> 3)) * p.HKV * kD * 2 + 16 * (lane & 7));
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int idx = r * 64 + lane;
+          const int tk = idx >> 4, vc = idx & 15;
+          vv[r >> 1][r & 1] = load16(vs_p, tk * p.HKV * kD * 2 + 16 * vc);
+        }
       }
     }
     }
@@ -941,19 +958,27 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
       else
         pv_loop(std::false_type());
     } else {
-      // contiguous layout: stage the V tile through LDS one half at a time ([64 tokens][64
-      // columns], a 132-byte row pitch keeps banks apart), then read columns (rows past the
-      // sequence end were loaded as zeros).  Half tiles keep two workgroups per CU in LDS.
-      uint8_t *st = s_vstage + wv * kPage * kVRowHalf;
+      // contiguous layout: stage the V tile through LDS some columns at a time (rows past the sequence end
+      // were loaded as zeros): half of them ([64 tokens][64 columns], a 136-byte row pitch keeps banks
+      // apart), so that two workgroups fit in a CU's LDS, or (many workgroups) a quarter, for three
+      uint8_t *st = s_vstage + wv * kPage * kVPitch;
+      constexpr int kPcs = kVCols / 8;  // 16-byte pieces of a staged row
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
+      for (int cf = 0; cf < kD / kVCols; ++cf) {
+        if constexpr (kBigC) {
+          if (cf == 2) {  // the last 64 columns, into the registers the first have freed
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int idx = r * 64 + lane;
-          const int tk = idx >> 4, vc = idx & 15;
-          if ((vc >> 3) == hf) {
+            for (int r = 0; r < 8; ++r)
+              vv[r >> 1][r & 1] = load16(vs_p, (8 * r + (lane >> 3)) * p.HKV * kD * 2 + 128 + 16 * (lane & 7));
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < (kBigC ? 8 : 16); ++r) {
+          const int tk = kBigC ? 8 * r + (lane >> 3) : (r * 64 + lane) >> 4;
+          const int vc = kBigC ? 8 * (cf >> 1) + (lane & 7) : lane & 15;  // 16-byte column piece
+          if (vc / kPcs == cf) {
             const uint4 v4 = vv[r >> 1][r & 1];
-            uint2 *d = (uint2 *)(st + tk * kVRowHalf + 16 * (vc & 7));  // rows are 8-byte aligned
+            uint2 *d = (uint2 *)(st + tk * kVPitch + 16 * (vc & (kPcs - 1)));  // rows are 8-byte aligned
             d[0] = make_uint2(v4.x, v4.y);
             d[1] = make_uint2(v4.z, v4.w);
           }
@@ -962,13 +987,13 @@ __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-        for (int nl = 0; nl < 4; ++nl) {
-          const int nu = 4 * hf + nl;
+        for (int nl = 0; nl < kVCols / 16; ++nl) {
+          const int nu = (kVCols / 16) * cf + nl;
 #pragma unroll
           for (int kap = 0; kap < 2; ++kap)
-            oacc[nu] = VTr::mfma(pa2[kap], VTr::operand(vt_operand_lds(st, kVRowHalf, nl, kap, kc, n)), oacc[nu]);
+            oacc[nu] = VTr::mfma(pa2[kap], VTr::operand(vt_operand_lds(st, kVPitch, nl, kap, kc, n)), oacc[nu]);
         }
-        // the other half (and the next kept chunk) reuses the staging buffer
+        // the next columns (and the next kept chunk) reuse the staging buffer
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -1402,6 +1427,23 @@ static hipError_t launch_decode(const ffa::DecodeParams &p, dim3 g0, hipStream_t
     const int cus = ffa::device_cus();
     if (p.span == ffa::kMinSpan && cus > 0 && grid.x * grid.y * grid.z <= (unsigned)cus) {
       hipLaunchKernelGGL((ffa::q2fp8_decode_2span_kernel<L, S, R, V>), grid, dim3(256), 0, st, p);
+      return hipGetLastError();
+    }
+  }
+  // contiguous per-channel with more workgroups than two per CU: the three-per-CU build.  Several quads of query rows
+  // per KV head share its data through the caches, and the second pass decides before it loads (64 query heads of 8,
+  // SBS 128: 8 x 16K tokens 175 -> 139 us, 4 x 64K 246 -> 175; with at most two per CU the sharing gave 1-2 %, and
+  // lost as much with mean values).  One quad: from five workgroups per CU on (32 query heads of 8: 8 x 16K 60.8 ->
+  // 58.9 us, 15 x 36K 164 -> 155); below that a third round of workgroups that is nearly empty costs more than the
+  // third resident one hides (4 layers of 2 x 30K, 944 workgroups: 127 -> 131; of 3 x 30K, 1416: 167 either way)
+  if constexpr (L == ffa::kContig && S == ffa::kChannel) {
+    const unsigned n = grid.x * grid.y * grid.z, cus = (unsigned)ffa::device_cus();
+    if (p.nq > 1 && cus > 0 && n > 2u * cus) {
+      hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, 3, true>), grid, dim3(256), 0, st, p);
+      return hipGetLastError();
+    }
+    if (p.nq == 1 && cus > 0 && n > 5u * cus) {
+      hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, 3, false>), grid, dim3(256), 0, st, p);
       return hipGetLastError();
     }
   }
