@@ -435,11 +435,13 @@ __global__ __launch_bounds__(512) void kproj_rope_kernel(const void *h, const vo
 //     steps ahead, one barrier a step; a step's operands are read under the products before them (with two
 //     buffers, and the reads and writes between the products, 57 us).  A row's eight pieces are stored at
 //     piece ^ (row & 7), so that the 16 rows an operand read touches spread over the banks (no conflicts).
-//   * Accumulators are folded into a second set every kGemmFold steps: chains as long as the split over
-//     eight waves gives at H = 4096, and its rounding error.
+//   * Accumulators are folded into a second set every eighth of K (512 of it at most): chains as long as the
+//     split over eight waves gives, and its rounding error (fp16 values that round otherwise than the 64-bit
+//     product, 4096 tokens: H = 1024 7.2e-4 of them with the split, 7.3e-4 here; H = 2048 9.4e-4 both, where
+//     folds every 512 gave 11.5e-4; H = 4096 12.3e-4 and 12.4e-4).
 //   * Workgroups go round-robin to the 8 XCDs; each XCD takes a run of consecutive tiles, channel tiles
 //     fastest, so that its L2 serves a tile row's tokens to every channel tile.
-constexpr int kGemmK = 64, kGemmFold = 8;
+constexpr int kGemmK = 64, kGemmMinH = 1024;
 
 template <int HDT, bool CS32, int TM, int TN>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void kproj_rope_tile_kernel(
@@ -559,11 +561,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1))) void k
   fetch(a1, b1, 3);
   lds_barrier();
   read(0, cur);
+  const int fold_mask = steps >= 64 ? 7 : (steps >= 32 ? 3 : 1);  // steps of a chain, less one
   int i = 0;
   for (; i + 1 < steps; i += 2) {
     step(a0, b0, i);
     step(a1, b1, i + 1);
-    if ((i & (kGemmFold - 1)) == kGemmFold - 2) fold();
+    if (((i + 2) & fold_mask) == 0) fold();
   }
   if (i < steps) step(a0, b0, i);
   fold();
@@ -963,8 +966,8 @@ static void launch_kproj_rope(const void *h, const void *w, const void *bias, co
   //   M = 2048   128x64 32, 64x64 36, 128x128 45, 128        M = 512    32x64 18, 64x64 20, 36
   // 32x64 tiles pay from half the CUs on (M = 256: 17.6 against 19.3; M = 128: 16.8 against 10.9).
   // Vector loads and stores need D and the pointers aligned, the K loop H a multiple of 64 (and a tile's rows
-  // within a buffer resource's 31 bits).
-  if (H % ffa::kGemmK == 0 && H < (1 << 22) && D % 4 == 0 && aligned(h, 16) && aligned(w, 16) && aligned(k_out, 16) &&
+  // within a buffer resource's 31 bits).  Below H = 1024 the split's chains are shorter than two steps.
+  if (H % ffa::kGemmK == 0 && H >= ffa::kGemmMinH && H < (1 << 22) && D % 4 == 0 && aligned(h, 16) && aligned(w, 16) && aligned(k_out, 16) &&
       aligned(cos, 16) && aligned(sin, 16)) {
     const int cus = ffa::device_cus() > 0 ? ffa::device_cus() : 256;
     auto tiles = [&](int tm, int tn) { return (long)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
