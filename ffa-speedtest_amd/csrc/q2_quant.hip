@@ -282,17 +282,20 @@ __device__ __forceinline__ uint4 kp_to_mfma_layout(uint4 v) {
                     (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)v.w));
 }
 
-// NB k steps of one wave: all 3 * NB loads are issued before the first MFMA waits.  They begin at step rot, another
-// one in each workgroup of an XCD: the rows' pitch is a power of two as a rule, and workgroups that walk it in
-// step ask the same few L2 channels at a time (64 tokens x 4096 -> 1024 with the append, 16 layers: 217 -> 207 us;
-// another start for each wave, which parts the neighbours that share 128-byte lines, 266).
+// NB k steps of one wave: all 3 * NB loads are issued before the first MFMA waits.  The column tiles of an XCD begin at
+// different steps, a quarter of the batch apart: the rows' pitch is a power of two as a rule, and workgroups that walk
+// it in step ask the same few L2 channels at a time (16 layers with the append, 1024 channels: 64 tokens of H = 2048
+// 167 -> 153 us, of H = 4096 227 -> 225, 256 tokens 403 -> 361; another start for each wave, which parts the
+// neighbours that share 128-byte lines, is slower).  The start depends on the output channels alone: with the token
+// tile in it as well 64 tokens of H = 4096 took 214, but a token's sums then depend on its row of the batch, and so
+// do its bytes in the cache.
 template <int NB, int HDT>
 __device__ __forceinline__ void kp_steps(const uint16_t *hp, const uint16_t *wp0, const uint16_t *wp1, int wv, int i,
-                                         int rot, f32x4 &acc0, f32x4 &acc1) {
+                                         int xcol, f32x4 &acc0, f32x4 &acc1) {
   uint4 a[NB], b0[NB], b1[NB];
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
-    const int k0 = 32 * (wv + kKpWaves * (i + ((j + rot) & (NB - 1))));
+    const int k0 = 32 * (wv + kKpWaves * (i + ((j + NB / 4 * xcol) & (NB - 1))));
     a[j] = *(const uint4 *)(hp + k0);
     b0[j] = *(const uint4 *)(wp0 + k0);
     b1[j] = *(const uint4 *)(wp1 + k0);
@@ -319,10 +322,10 @@ __device__ __forceinline__ float kproj_tile32(const void *h, const void *w, int 
   f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
   const int nsteps = H / 32;
   const int mine = (nsteps - wv + kKpWaves - 1) / kKpWaves;  // steps of this wave (16 at H = 4096)
-  const int rot = blockIdx.x >> 3;  // workgroups go round-robin to the 8 XCDs
+  const int xcol = n0 >> 8;  // which of its XCD's column tiles (they go round-robin to the 8 XCDs)
   int i = 0;
-  for (; i + 16 <= mine; i += 16) kp_steps<16, HDT>(hp, wp0, wp1, wv, i, rot, acc0, acc1);
-  for (; i + 4 <= mine; i += 4) kp_steps<4, HDT>(hp, wp0, wp1, wv, i, rot, acc0, acc1);
+  for (; i + 16 <= mine; i += 16) kp_steps<16, HDT>(hp, wp0, wp1, wv, i, xcol, acc0, acc1);
+  for (; i + 4 <= mine; i += 4) kp_steps<4, HDT>(hp, wp0, wp1, wv, i, xcol, acc0, acc1);
   for (; i < mine; ++i) kp_steps<1, HDT>(hp, wp0, wp1, wv, i, 0, acc0, acc1);
   // MFMA 16x16 result: acc[u] is row 4 * (lane >> 4) + u, column lane & 15
 #pragma unroll

@@ -165,6 +165,28 @@ def test_kproj_append_multi_token_bit_exact(gpu, B, Tn, H, use_bias):
             assert np.array_equal(v_pool[page, :, :, slot], vb[b, n]), ("V", b, n)
 
 
+@pytest.mark.parametrize("B,H,HKV", [(64, 4096, 8), (50, 2080, 4), (33, 512, 3)])
+def test_kproj_append_is_the_same_in_every_row(gpu, B, H, HKV):
+    """A token's K does not depend on its row of the batch: sequences with the same hidden state, position and angles
+    get the same bytes in every pool (H in whole batches of k steps and not, column tiles in and out of XCD order)."""
+    from ffa_mi355x import quant
+    from ffa_mi355x.paged import PagedQ2Cache
+
+    g = torch.Generator().manual_seed(H)
+    w = torch.randn(HKV * 128, H // 2, generator=g).bfloat16().repeat(1, 2).to(gpu)
+    x = torch.randn(H // 2, generator=g) * 100
+    # the halves cancel: what is left is the sums' own rounding, which another order would change
+    h = torch.cat([x, -x]).bfloat16().expand(B, 1, H).contiguous().to(gpu)
+    pos = torch.full((B,), 21, dtype=torch.int32, device=gpu)
+    bt = torch.arange(B, dtype=torch.int32, device=gpu)[:, None]
+    ang = (torch.rand(1, 1, 128, generator=g) * 6.28).expand(B, 1, 128).to(gpu)
+    cache = PagedQ2Cache(B, HKV, gpu)
+    quant.kproj_rope_q2_append(cache, h, w, ang.cos(), ang.sin(), pos, bt)
+    for pool in (cache.k_q, cache.k_scale, cache.k_zero, cache.k_res):
+        b = pool.view(torch.uint8)
+        assert bool((b == b[:1]).all()) and bool(b[0].any())
+
+
 def test_kproj_append_config5_small(gpu):
     """K-proj (theta 5e5, positions 65536+) + g32 quantize + paged append, then decode over the cache."""
     from ffa_mi355x import quant, synth
