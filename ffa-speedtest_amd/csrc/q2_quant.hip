@@ -747,6 +747,25 @@ __device__ __forceinline__ Raw8<DT> pack8(const float *x) {
   return r;
 }
 
+// 16 bytes of consecutive elements of kEs bytes at an address that is a multiple of 16 (WHOLE) or of kEs
+template <int kEs, bool WHOLE>
+__device__ __forceinline__ void store16(void *p, uint4 w) {
+  if constexpr (WHOLE) {
+    *(uint4 *)p = w;
+  } else {
+    const uint32_t v[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (kEs == 4) {
+        ((uint32_t *)p)[i] = v[i];
+      } else {
+        ((uint16_t *)p)[2 * i] = (uint16_t)(v[i] & 0xffffu);
+        ((uint16_t *)p)[2 * i + 1] = (uint16_t)(v[i] >> 16);
+      }
+    }
+  }
+}
+
 // Paged g32 cache -> contiguous K and V (the exact-attention path of the HF integration, which the
 // reference feeds with dequantized keys: ffa-fp8fp8/e2e/fp8fp8_cache.py:60-69, returned by update at
 // :84-89).  One workgroup per (sequence, page of the sequence, KV head): K = c * s + z + r in fp32
@@ -758,8 +777,9 @@ __device__ __forceinline__ Raw8<DT> pack8(const float *x) {
 // token 4 m + tau (residual blocks (tau, 0) and (tau, 1)), and V^T pieces of 8 tokens of one column.
 // Rows are put together in LDS and written 16 bytes a lane, whole rows at a time; V is turned by the
 // transposing LDS read (4 tokens x 32 columns per 16 lanes).  Written 2 bytes a lane at 64-byte distances,
-// as K and V were before, the cache of 4 sequences of 3K to 8K tokens, 214 MB, took 300 us; 56 now.
-template <bool E4M3, int VDT, int ODT>
+// as K and V were before, the cache of 4 sequences of 3K to 8K tokens, 214 MB, took 300 us; 56 now.  Outputs at
+// addresses that are no multiple of 16 bytes are written element by element (WHOLE = false).
+template <bool E4M3, int VDT, int ODT, bool WHOLE>
 __global__ __launch_bounds__(256) void q2_paged_dequant_kernel(const uint8_t *kq_pages, const uint16_t *s_pages,
                                                                const uint16_t *z_pages, const uint8_t *r_pages,
                                                                const uint16_t *v_pages, const int32_t *bt, int bt_stride,
@@ -817,7 +837,7 @@ __global__ __launch_bounds__(256) void q2_paged_dequant_kernel(const uint8_t *kq
   for (int i = 0; i < 64 * kPcs / 256; ++i) {
     const int tk = (threadIdx.x + 256 * i) / kPcs, q = threadIdx.x & (kPcs - 1);
     const uint4 w = *(const uint4 *)(s_t + tk * kRow + ((q ^ ((tk >> 2) & 7)) * 16));
-    *(uint4 *)((uint8_t *)k_out + (orow + (size_t)tk * HKV) * kRow + 16 * q) = w;
+    store16<kEs, WHOLE>((uint8_t *)k_out + (orow + (size_t)tk * HKV) * kRow + 16 * q, w);
   }
   __syncthreads();
 #pragma unroll
@@ -848,7 +868,8 @@ __global__ __launch_bounds__(256) void q2_paged_dequant_kernel(const uint8_t *kq
     const Raw8<ODT> o = pack8<ODT>(v);
 #pragma unroll
     for (int h = 0; h < kEs / 2; ++h)
-      *(uint4 *)((uint8_t *)v_out + (orow + (size_t)tk * HKV) * kRow + (32 * g + 8 * (x >> 2)) * kEs + 16 * h) = o.v[h];
+      store16<kEs, WHOLE>((uint8_t *)v_out + (orow + (size_t)tk * HKV) * kRow + (32 * g + 8 * (x >> 2)) * kEs + 16 * h,
+                          o.v[h]);
   }
 }
 }  // namespace ffa
@@ -1129,12 +1150,16 @@ extern "C" int ffa_q2_paged_dequant(const uint8_t *k_q_pages, const void *scale_
     return ffa_set_error_internal(FFA_E_INVALID, "null pointer");
   if (T % ffa::kPage) return ffa_set_error_internal(FFA_E_INVALID, "T must be a multiple of the 64-token page");
   const dim3 grid((unsigned)(T / ffa::kPage), (unsigned)HKV, (unsigned)B);
-#define FFA_CASE(EE, VV, OO)                                                                                         \
-  if ((res_dtype == FFA_DT_FP8_E4M3) == EE && v_dtype == VV && out_dtype == OO)                                      \
-    hipLaunchKernelGGL((ffa::q2_paged_dequant_kernel<EE, VV, OO>), grid, dim3(256), 0, (hipStream_t)stream,          \
+  const bool whole = aligned(k_out, 16) && aligned(v_out, 16);
+#define FFA_CASE(EE, VV, OO, WW)                                                                                     \
+  if ((res_dtype == FFA_DT_FP8_E4M3) == EE && v_dtype == VV && out_dtype == OO && whole == WW)                       \
+    hipLaunchKernelGGL((ffa::q2_paged_dequant_kernel<EE, VV, OO, WW>), grid, dim3(256), 0, (hipStream_t)stream,      \
                        k_q_pages, (const uint16_t *)scale_pages, (const uint16_t *)zero_pages, res_pages,            \
                        (const uint16_t *)v_pages, block_table, bt_stride, num_pages, seq_lens, T, HKV, k_out, v_out);
-#define FFA_CASES(EE, VV) FFA_CASE(EE, VV, FFA_DT_F16) FFA_CASE(EE, VV, FFA_DT_BF16) FFA_CASE(EE, VV, FFA_DT_F32)
+#define FFA_CASES(EE, VV)                                                      \
+  FFA_CASE(EE, VV, FFA_DT_F16, true) FFA_CASE(EE, VV, FFA_DT_F16, false)       \
+  FFA_CASE(EE, VV, FFA_DT_BF16, true) FFA_CASE(EE, VV, FFA_DT_BF16, false)     \
+  FFA_CASE(EE, VV, FFA_DT_F32, true) FFA_CASE(EE, VV, FFA_DT_F32, false)
   FFA_CASES(true, FFA_DT_F16)
   FFA_CASES(true, FFA_DT_BF16)
   FFA_CASES(false, FFA_DT_F16)

@@ -299,7 +299,8 @@ int ffa_q2_quantize_g32_append_cast(const void *k, int k_dtype, int B, int Tn, i
  * dequantized as k = c * scale + zero + residual (fp32, one rounding to out_dtype) and V copied
  * from the V^T pages (v_dtype F16/BF16).  T is a multiple of 64; tokens at or past seq_lens[b]
  * (seq_lens may be NULL: every sequence holds T tokens) are written as zeros.  Block-table
- * entries outside [0, num_pages) read page 0.  Feeds exact attention over the cache (prefill,
+ * entries outside [0, num_pages) read page 0.  k_out and v_out need the alignment of an element
+ * (multiples of 16 bytes are the fast case).  Feeds exact attention over the cache (prefill,
  * chunked prefill, and decode steps that do not prune).
  */
 int ffa_q2_paged_dequant(const uint8_t *k_q_pages, const void *scale_pages, const void *zero_pages,

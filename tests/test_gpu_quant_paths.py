@@ -218,6 +218,33 @@ def test_paged_dequantize_every_type(gpu, fmt, v_dt):
             assert torch.equal(x.cpu(), y.to(out))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("out", [torch.float32, torch.float16, torch.bfloat16])
+def test_paged_dequantize_into_any_address(gpu, out):
+    """Outputs at addresses that are multiples of an element's size alone (the C entry takes any) get the same values."""
+    from ffa_mi355x import _native as N
+    from ffa_mi355x.paged import PagedQ2Cache
+
+    B, HKV, T, lens = 2, 3, 128, torch.tensor([128, 65], dtype=torch.int32, device=gpu)
+    g = torch.Generator().manual_seed(6)
+    cache = PagedQ2Cache(B * 2, HKV, gpu)
+    bt = torch.arange(B * 2, dtype=torch.int32, device=gpu).view(B, 2)
+    k, v = (torch.randn(B, T, HKV, 128, generator=g).to(gpu) for _ in range(2))
+    cache.append(k, v, torch.zeros(B, dtype=torch.int32, device=gpu), bt)
+    want = cache.dequantize(bt, T, lens, out_dtype=out)
+    for ko, vo in ((1, 1), (0, 1), (3, 0)):
+        bufs = [torch.zeros(k.numel() + 8, dtype=out, device=gpu) for _ in range(2)]
+        got = [b[o:o + k.numel()] for b, o in zip(bufs, (ko, vo))]
+        N.check(N.lib().ffa_q2_paged_dequant(
+            cache.k_q.data_ptr(), cache.k_scale.data_ptr(), cache.k_zero.data_ptr(), cache.k_res.data_ptr(),
+            N.dtype_code(cache.res_dtype), cache.v.data_ptr(), N.dtype_code(cache.v_dtype), bt.data_ptr(), 2, B * 2,
+            lens.data_ptr(), B, T, HKV, got[0].data_ptr(), got[1].data_ptr(), N.dtype_code(out), N.stream_of(gpu)),
+            "ffa_q2_paged_dequant")
+        for x, y, b, o in zip(got, want, bufs, (ko, vo)):
+            assert torch.equal(x, y.reshape(-1))
+            assert not b[:o].any() and not b[o + k.numel():].any()
+
+
 # ------------------------------------------------------------------- paged appends
 def _pools(fmt, P, HKV, gpu, fill):
     """A cache whose bytes start as given, and its pools as bytes."""
