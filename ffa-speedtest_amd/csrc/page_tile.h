@@ -15,7 +15,7 @@
 namespace ffa {
 
 // V rows given with an append: how they are brought to the pool's 16-bit type (the conversions of a torch cast:
-// through fp32, round to nearest even).  Cast by the caller instead, 16K x 1024 bf16 values for an fp16 pool were
+// through fp32, round to nearest even, a NaN to bf16's 0x7fc0).  Cast by the caller instead, 16K x 1024 bf16 values for an fp16 pool were
 // 67 MB more to move, a launch and an allocation.
 enum { kVSame = 0, kVBf16ToF16 = 1, kVF16ToBf16 = 2, kVF32ToF16 = 3, kVF32ToBf16 = 4 };
 // element types (0 = f16, 1 = bf16, 2 = f32) of the rows and of the pool; -1: not one of the above
@@ -25,10 +25,17 @@ inline int v_mode(int from, int to) {
   if (from == 2) return to == 0 ? kVF32ToF16 : kVF32ToBf16;
   return from == 1 ? kVBf16ToF16 : (from == 0 ? kVF16ToBf16 : -1);
 }
+// a and b as the bf16 halves of a word, as a cast leaves them
+__device__ __forceinline__ uint32_t cast_pk_bf16(float a, float b) {
+  uint32_t w = pk_bf16_bits(a, b);
+  if (__builtin_isnan(a)) w = (w & 0xffff0000u) | 0x7fc0u;
+  if (__builtin_isnan(b)) w = (w & 0xffffu) | 0x7fc00000u;
+  return w;
+}
 __device__ __forceinline__ uint16_t v_element(const void *v, int vmode, size_t i) {
   if (vmode == kVSame) return ((const uint16_t *)v)[i];
   const float x = load_any(v, i, vmode == kVF16ToBf16 ? 0 : (vmode == kVBf16ToF16 ? 1 : 2));
-  return (uint16_t)(vmode == kVF16ToBf16 || vmode == kVF32ToBf16 ? f32_to_bf16_bits(x) : f32_to_f16_bits(x));
+  return (uint16_t)(vmode == kVF16ToBf16 || vmode == kVF32ToBf16 ? cast_pk_bf16(x, x) : f32_to_f16_bits(x));
 }
 
 struct PageTile {
@@ -111,7 +118,7 @@ __device__ __forceinline__ void page_tile_v(const void *v, int vmode, size_t row
         const bool bf = vmode == kVF16ToBf16 || vmode == kVF32ToBf16;
         uint32_t o[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = bf ? pk_bf16_bits(x[2 * e], x[2 * e + 1]) : pk_f16_bits(x[2 * e], x[2 * e + 1]);
+        for (int e = 0; e < 4; ++e) o[e] = bf ? cast_pk_bf16(x[2 * e], x[2 * e + 1]) : pk_f16_bits(x[2 * e], x[2 * e + 1]);
         w = make_uint4(o[0], o[1], o[2], o[3]);
       }
     }

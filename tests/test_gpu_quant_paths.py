@@ -246,12 +246,13 @@ def test_paged_dequantize_into_any_address(gpu, out):
 
 
 # ------------------------------------------------------------------- paged appends
-def _pools(fmt, P, HKV, gpu, fill):
+def _pools(fmt, P, HKV, gpu, fill, v_dtype=torch.float16):
     """A cache whose bytes start as given, and its pools as bytes."""
     from ffa_mi355x.paged import PagedQ2Cache
     from ffa_mi355x.paged_kfmt import PagedKfmtCache
 
-    c = PagedQ2Cache(P, HKV, gpu) if fmt == "q2" else PagedKfmtCache(fmt, P, HKV, gpu)
+    c = (PagedQ2Cache(P, HKV, gpu, v_dtype=v_dtype) if fmt == "q2" else
+         PagedKfmtCache(fmt, P, HKV, gpu, v_dtype=v_dtype))
     pools = [c.k_q, c.k_scale, c.k_zero, c.k_res, c.v] if fmt == "q2" else [c.k, c.k_scale, c.k_res, c.v]
     for t in pools:
         t.view(torch.uint8).fill_(fill)
@@ -330,6 +331,38 @@ def test_page_append_equals_token_append(gpu, fmt, k_dt, B, Tn, HKV, pos):
     for x, y in zip(wp, pp):
         assert np.array_equal(_u8(x), _u8(y))
     assert any((_u8(x) != 0x5A).any() for x in wp)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["q2", "nvfp4", "nf4"])
+@pytest.mark.parametrize("pool", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,Tn,HKV", [(2, 300, 9), (5, 1, 3)])  # whole pages for all formats; tokens for q2
+def test_append_casts_v_as_a_cast_does(gpu, fmt, pool, rows, B, Tn, HKV):
+    """V rows of another type than the pool's get the bytes of torch's cast, on the page and the per-token route:
+    ties, overflow, subnormals, infinities, NaNs of both signs among them."""
+    from ffa_mi355x.paged import VT_ORDER, to_logical
+
+    g = torch.Generator().manual_seed(Tn)
+    n = B * Tn * HKV * 128
+    bits = torch.randint(-2 ** 31, 2 ** 31, (n,), generator=g).to(torch.int32)  # every exponent, some NaNs
+    x = torch.where(torch.rand(n, generator=g) < 0.5, bits.view(torch.float32), torch.randn(n, generator=g))
+    inf, nan = float("inf"), float("nan")
+    x[:12] = torch.tensor([inf, -inf, nan, -nan, 65504.0, 65519.9, 65520.0, -65520.0, 2.0 ** -24, 2.0 ** -25, 3.39e38, 0.0])
+    x[12:14] = torch.tensor([0x3F808000, 0x3F818000], dtype=torch.int32).view(torch.float32)  # bf16 ties
+    v = x.view(B, Tn, HKV, 128).to(rows).to(gpu)
+    k = torch.randn(B, Tn, HKV, 128, generator=g).to(gpu)
+    npg = Tn // 64 + 2
+    bt = torch.randperm(B * npg, generator=g).view(B, npg).int()
+    pos = torch.tensor([(17 * b) % 64 for b in range(B)], dtype=torch.int32)
+    want = v.to(pool).view(torch.int16).cpu()
+    for keys in (k, _misaligned(k)):
+        cache, _ = _pools(fmt, B * npg, HKV, gpu, 0x5A, v_dtype=pool)
+        cache.append(keys, v, pos.to(gpu), bt.to(gpu))
+        got = to_logical(cache.v.view(torch.int16).cpu().numpy(), VT_ORDER)  # [P, HKV, 128, 64]
+        for b in range(B):
+            t = np.arange(Tn) + int(pos[b])
+            assert np.array_equal(got[bt[b].numpy()[t // 64], :, :, t % 64], want[b].numpy())
 
 
 # ------------------------------------------------------------------- nvfp4 / nf4 / fp8 in the reference layouts
