@@ -629,11 +629,12 @@ static int group_append(bool nf4, const void *k, int k_dtype, int B, int Tn, int
   if (bt_stride <= 0 || num_pages <= 0) return ffa_set_error_internal(FFA_E_INVALID, "empty block table or pool");
   if (!is_float(k_dtype)) return ffa_set_error_internal(FFA_E_INVALID, "k dtype");
   if (!is_fp8(res_dtype)) return ffa_set_error_internal(FFA_E_INVALID, "residual dtype must be fp8");
-  // Whole pages (16K tokens of one sequence: nvfp4 28 us against 154, nf4 35 against 160; one token of 64
-  // sequences 7.2 against 14.1 and 9.2 against 14.0, 4 of them 9.9 against 13.8 and equal) wherever K, V and
-  // the pools are aligned for 16-byte pieces and the tiles fit a grid dimension; the per-token kernel otherwise
-  if (ffa::page_tiles(Tn) <= 65535 && B <= 65535 && aligned(k, 16) && aligned(v_new, 16) && aligned(k_pages, 16) &&
-      aligned(res_pages, 16) && aligned(v_pages, 16) && aligned(scale_pages, 2)) {
+  // Whole pages (16K tokens of one sequence: nvfp4 28 us against 154, nf4 35 against 160) where the sizes favour them
+  // (k4_whole_pages), K, V and the pools are aligned for 16-byte pieces and the tiles fit a grid dimension; the
+  // per-token kernel otherwise
+  if (ffa::k4_whole_pages(nf4, B, Tn, HKV) && ffa::page_tiles(Tn) <= 65535 && B <= 65535 && aligned(k, 16) &&
+      aligned(v_new, 16) && aligned(k_pages, 16) && aligned(res_pages, 16) && aligned(v_pages, 16) &&
+      aligned(scale_pages, 2)) {
     const dim3 tiles((unsigned)HKV, (unsigned)ffa::page_tiles(Tn), (unsigned)B);
     const bool e4m3 = res_dtype == FFA_DT_FP8_E4M3;
 #define FFA_CASE(NN, KK, EE)                                                                                          \

@@ -11,6 +11,7 @@
 #pragma once
 
 #include "decode_common.h"
+#include "routes.h"
 
 namespace ffa {
 
@@ -56,8 +57,6 @@ __device__ __forceinline__ PageTile page_tile(const int32_t *pos, const int32_t 
   t.page = t.lo < t.hi ? append_page(bt, bt_stride, num_pages, b, t.P0) : -1;
   return t;
 }
-// tiles that Tn tokens at any position can touch
-inline int page_tiles(int Tn) { return (int)(((long)Tn + 126) >> 6); }
 
 constexpr int kVTilePitch = kVRow;  // LDS bytes of a V row
 template <int KDT>

@@ -1,0 +1,41 @@
+"""The rules by which calls choose between kernels that give the same bytes (csrc/routes.h), on the CPU: at the sizes
+where each kernel was measured to be the faster one, the rule takes it."""
+import shutil
+import subprocess
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+
+
+@pytest.fixture(scope="module")
+def routes(tmp_path_factory):
+    """routes(expression, ...): the values of C++ expressions over routes.h, as ints."""
+    cxx = shutil.which("g++") or shutil.which("clang++")
+    if cxx is None:
+        pytest.skip("no host compiler")
+    tmp = tmp_path_factory.mktemp("routes")
+
+    def run(*exprs):
+        src, exe = tmp / "r.cpp", tmp / "r"
+        body = "".join(f'  printf("%ld\\n", (long)({e}));\n' for e in exprs)
+        src.write_text('#include <stdio.h>\n#include "routes.h"\nusing namespace ffa;\nint main() {\n' + body + "}\n")
+        subprocess.run([cxx, "-std=c++17", f"-I{ROOT / 'ffa-speedtest_amd' / 'csrc'}", str(src), "-o", str(exe)], check=True)
+        return [int(x) for x in subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()]
+
+    return run
+
+
+def test_four_bit_appends(routes):
+    """Whole pages for few (sequence, head, page) blocks and for many tokens of each; the per-token kernel for a few
+    tokens of many sequences."""
+    nf4, nvfp4 = "true", "false"
+    whole = [(f, B, Tn, H) for f in (nf4, nvfp4) for B, Tn, H in
+             ((1, 1, 1), (64, 1, 8), (1, 4, 8), (1, 16384, 8), (4, 100, 4), (1024, 32, 1), (2048, 64, 16), (1, 2 ** 31 - 1, 8))]
+    whole += [(nvfp4, 1024, 1, 1), (nvfp4, 64, 4, 8), (nvfp4, 256, 16, 8), (nvfp4, 65536, 32, 64)]
+    tokens = [(f, B, Tn, H) for f in (nf4, nvfp4) for B, Tn, H in
+              ((2048, 2, 4), (512, 2, 16), (1024, 1, 4), (1024, 8, 2), (2048, 16, 1), (65535, 1, 1024))]
+    tokens += [(nf4, 256, 1, 8), (nf4, 512, 8, 8)]
+    got = routes(*(f"k4_whole_pages({f}, {B}, {Tn}, {H})" for f, B, Tn, H in whole + tokens))
+    assert got == [1] * len(whole) + [0] * len(tokens)
