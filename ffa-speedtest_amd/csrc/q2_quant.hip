@@ -1085,10 +1085,9 @@ static int q2_g32_append(const void *k, int k_dtype, int B, int Tn, int HKV, con
   if (!(res_dtype == FFA_DT_FP8_E4M3 || res_dtype == FFA_DT_FP8_E5M2))
     return ffa_set_error_internal(FFA_E_INVALID, "residual dtype must be fp8");
   const bool e4m3 = res_dtype == FFA_DT_FP8_E4M3;
-  // Whole pages from 32 tokens a sequence and 1024 in all (16K tokens of one sequence 29 us against 120, 4096
-  // 10 against 30, 512 equal, 16 x 32 tokens 6.5 against 6.0, one token of 64 sequences 6.4 against 3.6); the
-  // pieces need aligned rows and pools, the tiles are a grid dimension
-  if (Tn >= 32 && (long)B * Tn >= 1024 && ffa::page_tiles(Tn) <= 65535 && B <= 65535 && aligned(k, 16) &&
+  // Whole pages where the sizes favour them (q2_whole_pages); the pieces need aligned rows and pools, the tiles are a
+  // grid dimension
+  if (ffa::q2_whole_pages(B, Tn, HKV) && ffa::page_tiles(Tn) <= 65535 && B <= 65535 && aligned(k, 16) &&
       aligned(v_new, 16) && aligned(res_pages, 16) && aligned(v_pages, 16) && aligned(k_q_pages, 8)) {
     const dim3 grid((unsigned)HKV, (unsigned)ffa::page_tiles(Tn), (unsigned)B);
 #define FFA_CASE(KK, EE)                                                                                            \

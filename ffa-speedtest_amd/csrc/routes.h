@@ -6,6 +6,14 @@ namespace ffa {
 // pages that Tn tokens at any position can touch: workgroups of an append by whole pages, per sequence and KV head
 inline int page_tiles(int Tn) { return (int)(((long)Tn + 126) >> 6); }
 
+// 2-bit appends by whole (page, KV head) blocks rather than 128 threads per (token, head): for whole pages' worth of
+// tokens, from some 4600 rows (tokens x heads) on; below that a launch of either is all latency, 6 us against 3.5.  us,
+// per row against whole pages, fp16 V:
+//   rows 1024 (one head of 1024 tokens, 40 x 33)   4.5 / 6.5      2048   5.0 / 6.2      4096 (16 heads of 4 x 64, 4 of
+//   1024 tokens, 2 of 2048)   6.0 / 7.0, 6.5 / 6.8, 7.4 / 6.3     8192   9.1-11.6 / 6.6-8.3      16K tokens x 8 heads 120 / 29
+//   16 tokens a sequence, 8 and 16 heads   equal from 8192 rows on
+inline bool q2_whole_pages(int B, int Tn, int HKV) { return Tn >= 32 && (long)B * Tn * HKV >= 4608; }
+
 // nvfp4 / nf4 appends by whole (page, KV head) blocks rather than a thread per 16 channels of a token.  A workgroup of
 // the first costs some 6 ns (nvfp4; nf4 9) however few of its 64 slots it fills, past the 7 us that the smallest launch
 // takes; the second needs 14 us up to 8K rows (tokens x heads).  us, per token against whole pages, bf16 keys:

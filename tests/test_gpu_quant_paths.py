@@ -305,6 +305,10 @@ def test_nvfp4_and_nf4_code_turning_points():
     (2, 1025, 1, [1, 127]),
     (33, 32, 2, [7 * i for i in range(33)]),  # half a page each, across a page edge for some
     (5, 1, 2, [0, 1, 63, 64, 130]),       # single tokens (whole pages for the 4-bit formats only)
+    (1, 1024, 5, [0]),                    # the same with rows enough for the 2-bit pages
+    (1, 1100, 5, [63]),
+    (3, 1025, 2, [1, 127, 64]),
+    (33, 32, 5, [7 * i for i in range(33)]),
 ])
 def test_page_append_equals_token_append(gpu, fmt, k_dt, B, Tn, HKV, pos):
     """Appending whole pages writes the bytes that the per-token kernel (which takes keys at any address) writes, and

@@ -39,3 +39,11 @@ def test_four_bit_appends(routes):
     tokens += [(nf4, 256, 1, 8), (nf4, 512, 8, 8)]
     got = routes(*(f"k4_whole_pages({f}, {B}, {Tn}, {H})" for f, B, Tn, H in whole + tokens))
     assert got == [1] * len(whole) + [0] * len(tokens)
+
+
+def test_two_bit_appends(routes):
+    """Whole pages from about 4600 rows (tokens x heads) on, of 32 tokens a sequence or more."""
+    whole = [(1, 16384, 8), (1, 1024, 8), (2, 3000, 4), (144, 32, 1), (1, 8192, 1), (1, 2 ** 31 - 1, 64)]
+    tokens = [(1, 1024, 1), (40, 33, 1), (4, 64, 16), (1, 512, 8), (64, 1, 8), (4096, 31, 8), (65535, 1, 64)]
+    got = routes(*(f"q2_whole_pages({B}, {Tn}, {H})" for B, Tn, H in whole + tokens))
+    assert got == [1] * len(whole) + [0] * len(tokens)
