@@ -984,25 +984,16 @@ static void launch_kproj_tile(const void *h, const void *w, const void *bias, co
 template <int HDT>
 static void launch_kproj_rope(const void *h, const void *w, const void *bias, const void *cos, const void *sin, int csdt,
                               int M, int T, int H, int N, int D, void *k_out, int odt, hipStream_t st) {
-  // The largest tile that still gives every CU a workgroup (us at H = 4096, N = 1024, bf16; the 16 x 32 tiles
-  // of kproj_rope_kernel last):
-  //   M = 4096   128x128 53, 128x64 57, 64x64 72, 249        M = 1024   64x64 22, 32x64 26, 128x64 30, 67
-  //   M = 2048   128x64 32, 64x64 36, 128x128 45, 128        M = 512    32x64 18, 64x64 20, 36
-  // 32x64 tiles pay from half the CUs on (M = 256: 17.6 against 19.3; M = 128: 16.8 against 10.9).
   // Vector loads and stores need D and the pointers aligned, the K loop H a multiple of 64 (and a tile's rows
   // within a buffer resource's 31 bits).  Below H = 1024 the split's chains are shorter than two steps.
-  if (H % ffa::kGemmK == 0 && H >= ffa::kGemmMinH && H < (1 << 22) && D % 4 == 0 && aligned(h, 16) && aligned(w, 16) && aligned(k_out, 16) &&
-      aligned(cos, 16) && aligned(sin, 16)) {
-    const int cus = ffa::device_cus() > 0 ? ffa::device_cus() : 256;
-    auto tiles = [&](int tm, int tn) { return (long)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
-    if (tiles(128, 128) >= cus)
-      return launch_kproj_tile<HDT, 128, 128>(h, w, bias, cos, sin, csdt, M, T, H, N, D, k_out, st);
-    if (tiles(128, 64) >= cus)
-      return launch_kproj_tile<HDT, 128, 64>(h, w, bias, cos, sin, csdt, M, T, H, N, D, k_out, st);
-    if (tiles(64, 64) >= cus)
-      return launch_kproj_tile<HDT, 64, 64>(h, w, bias, cos, sin, csdt, M, T, H, N, D, k_out, st);
-    if (tiles(32, 64) >= cus / 2)
-      return launch_kproj_tile<HDT, 32, 64>(h, w, bias, cos, sin, csdt, M, T, H, N, D, k_out, st);
+  if (H % ffa::kGemmK == 0 && H >= ffa::kGemmMinH && H < (1 << 22) && D % 4 == 0 && aligned(h, 16) && aligned(w, 16) &&
+      aligned(k_out, 16) && aligned(cos, 16) && aligned(sin, 16)) {
+    switch (ffa::kproj_route(M, N, ffa::device_cus() > 0 ? ffa::device_cus() : 256)) {
+      case ffa::kKproj128x128: return launch_kproj_tile<HDT, 128, 128>(h, w, bias, cos, sin, csdt, M, T, H, N, D, k_out, st);
+      case ffa::kKproj128x64: return launch_kproj_tile<HDT, 128, 64>(h, w, bias, cos, sin, csdt, M, T, H, N, D, k_out, st);
+      case ffa::kKproj64x64: return launch_kproj_tile<HDT, 64, 64>(h, w, bias, cos, sin, csdt, M, T, H, N, D, k_out, st);
+      case ffa::kKproj32x64: return launch_kproj_tile<HDT, 32, 64>(h, w, bias, cos, sin, csdt, M, T, H, N, D, k_out, st);
+    }
   }
   hipLaunchKernelGGL(ffa::kproj_rope_kernel<HDT>, dim3((unsigned)((N / 32) * ((M + 15) / 16))), dim3(512), 0, st, h, w,
                      bias, cos, sin, csdt, M, T, H, N, D, k_out, odt);

@@ -27,4 +27,26 @@ inline bool k4_whole_pages(bool nf4, int B, int Tn, int HKV) {
   return workgroups <= (nf4 ? 512 : 1024) || Tn >= 32 || (!nf4 && Tn >= 16 && HKV >= 8);
 }
 
+// K projection + RoPE of M tokens onto N channels: the split kernel (16 tokens x 32 channels a workgroup) or a tile of
+// the LDS-staged one.  us at H = 4096, bf16 (the order is the same from H = 1024 to 8192):
+//   N = 1024, tiles 128x128 / 128x64 / 64x64 / 32x64, split
+//     M = 256  - / - / 21 / 18, 18    512  45 / 31 / 22 / 18, 36    1024  45 / 32 / 22 / 26, 67    2048  45 / 32 / 36 / -, 128
+//     4096  53 / 57 / 72 / -, 249    4100  87 / 70 / 70 / -, 230    5200  89 / 73 / 85 / -, 287    8200  130 / 112 / -, 447
+//   N = 32 (half of a tile's channels unused)   M = 4096  32x64 17.3, split 11.7    4224  17.2, 18.8    5200  17.7, 19.5
+//   N = 2048   M = 100  32x64 18.0, split 16.5    128  18.1, 17.3      N = 8192   M = 32  17.8, 26.6    100  42.6, 80.6
+// So: the split kernel while its workgroups are one round (a few more than one a CU run beside the others), for short
+// prompts up to N = 2048, and where the smallest tiles fill less than half the chip; then the largest tile that gives
+// every CU a workgroup.  A 128x128 workgroup has its CU to itself, so a last round of them that is at most half full costs as much
+// as a full one: 128x64 tiles take it, two a CU, where their number is whole in XCD order (elsewhere they were the
+// slower ones: M = 12000, N = 384 95 -> 109).
+enum { kKprojSplit = 0, kKproj32x64, kKproj64x64, kKproj128x64, kKproj128x128 };
+inline int kproj_route(int M, int N, int cus) {
+  auto tiles = [&](int tm, int tn) { return (long)((M + tm - 1) / tm) * ((N + tn - 1) / tn); };
+  const long split = (long)((M + 15) / 16) * (N / 32);
+  if (tiles(32, 64) < cus / 2 || split < cus + cus / 32 || (M <= 128 && N <= 2048)) return kKprojSplit;
+  const long large = tiles(128, 128), over = large % cus;
+  if (large >= cus) return over > 0 && 2 * over <= cus && tiles(128, 64) % 8 == 0 ? kKproj128x64 : kKproj128x128;
+  return tiles(128, 64) >= cus ? kKproj128x64 : (tiles(64, 64) >= cus ? kKproj64x64 : kKproj32x64);
+}
+
 }  // namespace ffa

@@ -127,9 +127,10 @@ def test_q2_quantizer_vector_route_equals_scalar_route(gpu, tau, B, T, HKV, D):
 @pytest.mark.gpu
 @pytest.mark.parametrize("h_dt", ["bf16", "fp16"])
 @pytest.mark.parametrize("B,T,HKV,D,H,cs32,bias", [
-    (1, 4100, 8, 128, 1088, True, False),   # 128 x 128 tiles (33 x 8), 17 steps folded by 2, ragged last tile row
+    (1, 4100, 8, 128, 1088, True, False),   # 128 x 64 tiles (33 x 16), 17 steps folded by 2, ragged last tile row
+    (1, 6200, 8, 128, 1088, True, False),   # 128 x 128 (49 x 8), the same
     (2, 2048, 8, 128, 2112, False, True),   # 128 x 128, 33 steps folded by 4, two sequences
-    (1, 4200, 35, 32, 1216, True, True),    # 128 x 128, a ragged last column of tiles, grid not a multiple of 8
+    (1, 4200, 35, 32, 1216, True, True),    # 128 x 128 (33 x 9), a ragged last column, grid not a multiple of 8
     (3, 700, 8, 128, 4160, True, True),     # 128 x 64 (17 x 16), 65 steps folded by 8
     (1, 1030, 8, 128, 1024, False, False),  # 64 x 64 (17 x 16), the shortest K of the tiles
     (1, 290, 7, 128, 1152, True, False),    # 32 x 64 (10 x 14)

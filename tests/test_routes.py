@@ -47,3 +47,14 @@ def test_two_bit_appends(routes):
     tokens = [(1, 1024, 1), (40, 33, 1), (4, 64, 16), (1, 512, 8), (64, 1, 8), (4096, 31, 8), (65535, 1, 64)]
     got = routes(*(f"q2_whole_pages({B}, {Tn}, {H})" for B, Tn, H in whole + tokens))
     assert got == [1] * len(whole) + [0] * len(tokens)
+
+
+def test_projection_tiles(routes):
+    """Each tile, and the split kernel, where it was measured to be the fastest (256 CUs)."""
+    want = {"kKprojSplit": [(64, 1024), (128, 1024), (4096, 32), (4100, 32), (100, 2048), (128, 2048), (1, 32), (16, 8192)],
+            "kKproj32x64": [(32, 8192), (64, 4096), (256, 1024), (512, 1024), (4096, 64), (5200, 32), (2048, 128)],
+            "kKproj64x64": [(1024, 1024), (1100, 1024)],
+            "kKproj128x64": [(2048, 1024), (2100, 1024), (4100, 1024), (4224, 1024), (5200, 1024), (8200, 1024)],
+            "kKproj128x128": [(4096, 1024), (4096 + 128 * 17, 1024), (8192, 1024), (12000, 384), (1 << 22, 1024)]}
+    for tile, sizes in want.items():
+        assert routes(*(f"kproj_route({M}, {N}, 256) == {tile}" for M, N in sizes)) == [1] * len(sizes), tile
