@@ -16,6 +16,7 @@
 #include "page_tile.h"
 
 #include <stdio.h>
+#include <type_traits>
 
 #pragma clang fp contract(off)
 
@@ -289,13 +290,13 @@ __device__ __forceinline__ uint4 kp_to_mfma_layout(uint4 v) {
 // neighbours that share 128-byte lines, is slower).  The start depends on the output channels alone: with the token
 // tile in it as well 64 tokens of H = 4096 took 214, but a token's sums then depend on its row of the batch, and so
 // do its bytes in the cache.
-template <int NB, int HDT>
+template <int NB, int HDT, bool kFirst>
 __device__ __forceinline__ void kp_steps(const uint16_t *hp, const uint16_t *wp0, const uint16_t *wp1, int wv, int i,
                                          int xcol, f32x4 &acc0, f32x4 &acc1) {
   uint4 a[NB], b0[NB], b1[NB];
 #pragma unroll
   for (int j = 0; j < NB; ++j) {
-    const int k0 = 32 * (wv + kKpWaves * (i + ((j + NB / 4 * xcol) & (NB - 1))));
+    const int k0 = 32 * (wv + kKpWaves * (i + (kFirst ? j : (j + NB / 4 * xcol) & (NB - 1))));
     a[j] = *(const uint4 *)(hp + k0);
     b0[j] = *(const uint4 *)(wp0 + k0);
     b1[j] = *(const uint4 *)(wp1 + k0);
@@ -323,10 +324,16 @@ __device__ __forceinline__ float kproj_tile32(const void *h, const void *w, int 
   const int nsteps = H / 32;
   const int mine = (nsteps - wv + kKpWaves - 1) / kKpWaves;  // steps of this wave (16 at H = 4096)
   const int xcol = n0 >> 8;  // which of its XCD's column tiles (they go round-robin to the 8 XCDs)
-  int i = 0;
-  for (; i + 16 <= mine; i += 16) kp_steps<16, HDT>(hp, wp0, wp1, wv, i, xcol, acc0, acc1);
-  for (; i + 4 <= mine; i += 4) kp_steps<4, HDT>(hp, wp0, wp1, wv, i, xcol, acc0, acc1);
-  for (; i < mine; ++i) kp_steps<1, HDT>(hp, wp0, wp1, wv, i, 0, acc0, acc1);
+  // the first column tile of an XCD begins at step 0: addresses without arithmetic (1024 x 4096 -> 64 10.1 -> 9.7 us)
+  auto steps = [&](auto first) {
+    constexpr bool kFirst = decltype(first)::value;
+    int i = 0;
+    for (; i + 16 <= mine; i += 16) kp_steps<16, HDT, kFirst>(hp, wp0, wp1, wv, i, xcol, acc0, acc1);
+    for (; i + 4 <= mine; i += 4) kp_steps<4, HDT, kFirst>(hp, wp0, wp1, wv, i, xcol, acc0, acc1);
+    for (; i < mine; ++i) kp_steps<1, HDT, true>(hp, wp0, wp1, wv, i, 0, acc0, acc1);
+  };
+  if (xcol == 0) steps(std::true_type());
+  else steps(std::false_type());
   // MFMA 16x16 result: acc[u] is row 4 * (lane >> 4) + u, column lane & 15
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
