@@ -38,6 +38,7 @@
 //     residual/V traffic spreads over every XCD's memory path.
 #include "decode_common.h"
 #include "ffa_mi355x.h"
+#include "routes.h"
 
 #include <stdio.h>
 
@@ -145,9 +146,9 @@ __host__ __device__ constexpr int scale_pos(int t) { return 16 * (t >> 4) + 4 * 
 // waves 0 and 1, which would own none, load the residual and V rows of chunk wv (the chunk of wave
 // wv + 2) right after the operand barrier, before the prune decides it, and refine that chunk from
 // their registers if it is kept.
-// SHARE (several quads of query rows per KV head; paged g32, contiguous per-channel): the quads' workgroups read the
-// same codes, scales, residual and V from the caches (paged: from one XCD's L2, decode_unit), so these loads keep
-// the default cache policy (bload16_nt's, for data that one workgroup reads: 68.5 against 62.8 us for 8 sequences
+// SHARE (several quads of query rows per KV head; paged g32 where quads_share says so, contiguous per-channel): the
+// quads' workgroups read the same codes, scales, residual and V from the caches (paged: with 8 or 16 KV heads from one
+// XCD's L2, decode_unit), so these loads keep the default cache policy (bload16_nt's, for data that one workgroup reads: 68.5 against 62.8 us for 8 sequences
 // of 3K-16K tokens with 64 query heads; one quad without the hint, 32K tokens, 16 layers: 219 against 204 us).
 template <int LAYOUT, int SMODE, int RES, int VT, int OCC, bool SPEC, bool SHARE>
 __device__ __forceinline__ void q2fp8_decode_body(const DecodeParams &p) {
@@ -1410,7 +1411,7 @@ static hipError_t launch_decode(const ffa::DecodeParams &p, dim3 g0, hipStream_t
   if constexpr (L == ffa::kPaged && S == ffa::kG32) {
     const int cus = ffa::device_cus();
     const bool many = cus > 0 && grid.x * grid.y * grid.z > 2u * (unsigned)cus;
-    if (p.nq > 1) {  // several quads of query rows per KV head share its data
+    if (ffa::quads_share(p.nq, p.HKV, (long)grid.x * grid.y * grid.z, cus)) {
       if (many)
         hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, 4, true>), grid, dim3(256), 0, st, p);
       else

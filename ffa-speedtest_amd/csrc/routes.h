@@ -27,6 +27,18 @@ inline bool k4_whole_pages(bool nf4, int B, int Tn, int HKV) {
   return workgroups <= (nf4 ? 512 : 1024) || Tn >= 32 || (!nf4 && Tn >= 16 && HKV >= 8);
 }
 
+// Paged 2-bit decode with nq quads of query rows per KV head: whether the quads' loads keep the default cache policy and
+// pass 2 decides before it loads (the SHARE builds).  With a multiple of 8 KV heads the quads of one run on one XCD; one
+// head's few workgroups gain as well.  Elsewhere the quads meet in the last-level cache only, which pays where rounds of
+// workgroups queue up: time over that of the other builds, groups of 8, at a usual and a full share of kept blocks
+//   4 heads  one a CU (16K tokens) 0.98, 1.05    2.25 a CU (4 x 3K-9K) 1.02, 1.02    3 (50K) 0.92, 0.97    6 (100K) 0.81, 0.95
+//   2 heads  one a CU (32K) 0.96, 1.04 (groups of 5 1.00, 1.10)    1.5 (50K) 0.95, 1.02    3 (100K) 0.93, 1.00
+//   3 heads  0.75 a CU (16K) 0.97, 1.06    2.3 (50K) 0.94, 0.98    2.6 (4 x 14K) 0.91, 0.98
+//   1 head   up to 1.5 a CU 0.96-1.00      8 heads  2 a CU (32K) 0.92, 0.77 of the build without this unit order
+inline bool quads_share(int nq, int HKV, long workgroups, int cus) {
+  return nq > 1 && (HKV % 8 == 0 || HKV == 1 || 2 * workgroups > 5 * (long)cus);
+}
+
 // K projection + RoPE of M tokens onto N channels: the split kernel (16 tokens x 32 channels a workgroup) or a tile of
 // the LDS-staged one.  us at H = 4096, bf16 (the order is the same from H = 1024 to 8192):
 //   N = 1024, tiles 128x128 / 128x64 / 64x64 / 32x64, split

@@ -58,3 +58,11 @@ def test_projection_tiles(routes):
             "kKproj128x128": [(4096, 1024), (4096 + 128 * 17, 1024), (8192, 1024), (12000, 384), (1 << 22, 1024)]}
     for tile, sizes in want.items():
         assert routes(*(f"kproj_route({M}, {N}, 256) == {tile}" for M, N in sizes)) == [1] * len(sizes), tile
+
+
+def test_decode_of_several_quads(routes):
+    """Quads of a KV head share its data with 8 or 16 heads or one, and in grids of more than 2.5 workgroups a CU."""
+    share = [(2, 8, 128), (4, 16, 10000), (2, 1, 64), (4, 1, 2000), (2, 4, 784), (2, 3, 672), (2, 2, 641)]
+    apart = [(1, 8, 100000), (1, 1, 10), (2, 4, 256), (2, 4, 576), (2, 2, 256), (2, 3, 384), (4, 6, 640)]
+    got = routes(*(f"quads_share({nq}, {H}, {n}, 256)" for nq, H, n in share + apart))
+    assert got == [1] * len(share) + [0] * len(apart)
