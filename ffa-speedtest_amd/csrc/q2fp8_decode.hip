@@ -1431,20 +1431,15 @@ static hipError_t launch_decode(const ffa::DecodeParams &p, dim3 g0, hipStream_t
       return hipGetLastError();
     }
   }
-  // contiguous per-channel with more workgroups than two per CU: the three-per-CU build.  Several quads of query rows
-  // per KV head share its data through the caches, and the second pass decides before it loads (64 query heads of 8,
-  // SBS 128: 8 x 16K tokens 175 -> 139 us, 4 x 64K 246 -> 175; with at most two per CU the sharing gave 1-2 %, and
-  // lost as much with mean values).  One quad: from five workgroups per CU on (32 query heads of 8: 8 x 16K 60.8 ->
-  // 58.9 us, 15 x 36K 164 -> 155); below that a third round of workgroups that is nearly empty costs more than the
-  // third resident one hides (4 layers of 2 x 30K, 944 workgroups: 127 -> 131; of 3 x 30K, 1416: 167 either way)
+  // contiguous per-channel, many workgroups: the three-per-CU build.  Several quads of query rows per KV head share its
+  // data through the caches, and the second pass decides before it loads
   if constexpr (L == ffa::kContig && S == ffa::kChannel) {
-    const unsigned n = grid.x * grid.y * grid.z, cus = (unsigned)ffa::device_cus();
-    if (p.nq > 1 && cus > 0 && n > 2u * cus) {
-      hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, 3, true>), grid, dim3(256), 0, st, p);
-      return hipGetLastError();
-    }
-    if (p.nq == 1 && cus > 0 && n > 5u * cus) {
-      hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, 3, false>), grid, dim3(256), 0, st, p);
+    const int cus = ffa::device_cus();
+    if (cus > 0 && ffa::three_per_cu(p.nq, (long)grid.x * grid.y * grid.z, cus, p.delta)) {
+      if (p.nq > 1)
+        hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, 3, true>), grid, dim3(256), 0, st, p);
+      else
+        hipLaunchKernelGGL((ffa::q2fp8_decode_kernel<L, S, R, V, 3, false>), grid, dim3(256), 0, st, p);
       return hipGetLastError();
     }
   }

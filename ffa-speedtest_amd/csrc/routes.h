@@ -39,6 +39,21 @@ inline bool quads_share(int nq, int HKV, long workgroups, int cus) {
   return nq > 1 && (HKV % 8 == 0 || HKV == 1 || 2 * workgroups > 5 * (long)cus);
 }
 
+// Contiguous per-channel 2-bit decode: whether the build for three workgroups per CU is taken (V staged a quarter of its
+// columns at a time) or that for two.
+// Several quads per KV head, from more than two workgroups a CU: 8 x 16K tokens, 64 query heads of 8, 175 -> 139 us,
+// 4 x 64K 246 -> 175, and faster at every share of kept blocks (0.80-0.99); with at most two a CU the sharing that comes
+// with it gave 1-2 %, and lost as much with mean values.
+// One quad, from five a CU: below that a third round of workgroups that is nearly empty costs more than the third
+// resident one hides (4 layers of 2 x 30K, 944 workgroups: 127 -> 131 us; of 3 x 30K, 1416: 167 either way).  It pays
+// while pruned chunks leave the CUs waiting: 8 x 16K to 32 x 16K tokens, 32 query heads of 8, 0.94-0.95 of the time at
+// 40 % of the blocks kept, 0.99-1.02 at 70 %, but 1.06-1.10 with all of them, where the narrower staging shows (with
+// mean values 0.94-0.95, 0.95-0.98, 0.97-1.04).  The threshold's distance from the probes' maximum is what a launch
+// knows of that: with the usual 5 or less the three-per-CU build (at 8 the ratios are 0.89 to 1.03).
+inline bool three_per_cu(int nq, long workgroups, int cus, float delta) {
+  return nq > 1 ? workgroups > 2 * (long)cus : workgroups > 5 * (long)cus && delta <= 5.f;
+}
+
 // K projection + RoPE of M tokens onto N channels: the split kernel (16 tokens x 32 channels a workgroup) or a tile of
 // the LDS-staged one.  us at H = 4096, bf16 (the order is the same from H = 1024 to 8192):
 //   N = 1024, tiles 128x128 / 128x64 / 64x64 / 32x64, split

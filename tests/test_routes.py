@@ -66,3 +66,12 @@ def test_decode_of_several_quads(routes):
     apart = [(1, 8, 100000), (1, 1, 10), (2, 4, 256), (2, 4, 576), (2, 2, 256), (2, 3, 384), (4, 6, 640)]
     got = routes(*(f"quads_share({nq}, {H}, {n}, 256)" for nq, H, n in share + apart))
     assert got == [1] * len(share) + [0] * len(apart)
+
+
+def test_contiguous_decode_of_many_workgroups(routes):
+    """Three workgroups a CU: several quads from more than two a CU on, one quad from more than five where the threshold
+    lies near the maximum."""
+    three = [(2, 513, 5.0), (4, 100000, 1000.0), (1, 1281, 5.0), (1, 8520, 0.0)]
+    two = [(2, 512, 5.0), (1, 1280, 5.0), (1, 944, 5.0), (1, 8520, 8.0), (1, 8520, 1000.0)]
+    got = routes(*(f"three_per_cu({nq}, {n}, 256, {d}f)" for nq, n, d in three + two))
+    assert got == [1] * len(three) + [0] * len(two)
