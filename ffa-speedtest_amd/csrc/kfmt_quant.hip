@@ -148,7 +148,8 @@ __device__ __forceinline__ void fp4_levels8(uint32_t w, float *l) {
   l[0] = a[0], l[1] = a[1], l[2] = b[0], l[3] = b[1], l[4] = c[0], l[5] = c[1], l[6] = d[0], l[7] = d[1];
 }
 
-// The same over vectors of 8 channels (D a multiple of 8, aligned pointers).  A page's K is read once: up to
+// The same over vectors of 8 channels (D a multiple of 8, aligned pointers, pages that fill the threads:
+// nvfp4_by_vectors).  A page's K is read once: up to
 // kHold vectors a thread stay in registers from the maximum to the codes (a page of 128 tokens x 128 channels
 // in 16 bits), longer pages are read again.  The codes come by comparison: the scale is one value for the whole
 // workgroup, so where tau(|k| / scale) passes an e2m1 midpoint is seven floats, worked out once (fp4_turn), in
@@ -578,7 +579,7 @@ extern "C" int ffa_nvfp4_quantize(const void *k, int k_dtype, int B, int T, int 
   if (!is_float(k_dtype)) return ffa_set_error_internal(FFA_E_INVALID, "k dtype");
   if (!is_fp8(res_dtype)) return ffa_set_error_internal(FFA_E_INVALID, "residual dtype must be fp8");
   const int npg = (T + page_size - 1) / page_size;
-  if (D % 8 == 0 && aligned(k, 16) && aligned(residual, 8) && aligned(k_packed, 4)) {
+  if (ffa::nvfp4_by_vectors(D, page_size) && aligned(k, 16) && aligned(residual, 8) && aligned(k_packed, 4)) {
     const bool e4m3 = res_dtype == FFA_DT_FP8_E4M3;
 #define FFA_CASE(KK, EE)                                                                                              \
   if (k_dtype == KK && e4m3 == EE)                                                                                    \

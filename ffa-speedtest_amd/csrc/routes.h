@@ -6,6 +6,11 @@ namespace ffa {
 // pages that Tn tokens at any position can touch: workgroups of an append by whole pages, per sequence and KV head
 inline int page_tiles(int Tn) { return (int)(((long)Tn + 126) >> 6); }
 
+// nvfp4 quantizer of the reference layout by vectors of 8 channels, a page of a KV head per workgroup: pages of more than
+// 256 values.  Smaller ones leave most of its threads without a vector (time over the element-wise kernel's, 16-bit keys
+// of 30K tokens: 64 values 1.3-1.5, 128 1.2-1.4, 256 0.9-1.06, 384 0.8-0.9, 8192 0.3).
+inline bool nvfp4_by_vectors(int D, int page) { return D % 8 == 0 && (long)D * page > 256; }
+
 // 2-bit appends by whole (page, KV head) blocks rather than 128 threads per (token, head): for whole pages' worth of
 // tokens, from some 4600 rows (tokens x heads) on; below that a launch of either is all latency, 6 us against 3.5.  us,
 // per row against whole pages, fp16 V:

@@ -60,6 +60,13 @@ def test_projection_tiles(routes):
         assert routes(*(f"kproj_route({M}, {N}, 256) == {tile}" for M, N in sizes)) == [1] * len(sizes), tile
 
 
+def test_nvfp4_vectors(routes):
+    """Vectors of 8 channels for pages of more than 256 values."""
+    vectors, scalar = [(128, 128), (8, 33), (24, 16), (8, 2 ** 31 - 1)], [(8, 16), (16, 16), (128, 2), (12, 128), (1, 1000)]
+    got = routes(*(f"nvfp4_by_vectors({D}, {page})" for D, page in vectors + scalar))
+    assert got == [1] * len(vectors) + [0] * len(scalar)
+
+
 def test_decode_of_several_quads(routes):
     """Quads of a KV head share its data with 8 or 16 heads or one, and in grids of more than 2.5 workgroups a CU."""
     share = [(2, 8, 128), (4, 16, 10000), (2, 1, 64), (4, 1, 2000), (2, 4, 784), (2, 3, 672), (2, 2, 641)]
