@@ -33,7 +33,9 @@ from . import _native as N
 from .decode import HEAD_DIM, DecodeWorkspace, run_decode
 
 PAGE = 64
-_CHECK_ON_HOST = 16384  # block-table entries (64 KB) that an append's bounds check copies whole
+# Block-table entries up to which an append's bounds check copies the table whole rather than reducing it where it lies
+# (us of a check, copied / reduced: up to 256 entries 26 / 70, 16384 35 / 71-79, 65536 43-46 / 77-79, 262144 98-126 / 80-84)
+_CHECK_ON_HOST = 65536
 
 
 def _orders():
