@@ -119,7 +119,7 @@ def test_reference_smoke_test(gpu):
 def test_kproj_append_multi_token_bit_exact(gpu, B, Tn, H, use_bias):
     """Appends of several tokens per sequence (token tiles with a ragged last tile, page boundaries,
     H with whole and partial k batches, bias): every byte equals the oracle's g32 quantization of the
-    rotated K that ffa_kproj_rope (the same GEMM tile) computes; V^T bytes are the new V."""
+    rotated K that ffa_kproj_rope (for so few tokens the same GEMM tile) computes; V^T bytes are the new V."""
     from ffa_mi355x import kfmt_quant as KQ
     from ffa_mi355x import quant, synth
     from ffa_mi355x.paged import CODES_ORDER, GSCALE_ORDER, RES_ORDER, VT_ORDER, PagedQ2Cache, to_logical
@@ -230,7 +230,7 @@ def test_kproj_append_config5_small(gpu):
         vg = v_pool[page, :, :, slot]
         assert torch.equal(vg, v_new[b, 0])
     assert mism <= 0.01 * B * HKV * 128
-    # ffa_kproj_rope runs the same GEMM tile (same fp32 sums), so its rotated K, quantized by the oracle,
+    # ffa_kproj_rope runs the same GEMM tile for so few tokens (same fp32 sums), so its rotated K, quantized by the oracle,
     # must give exactly the appended bytes
     from ffa_mi355x import kfmt_quant as KQ
 

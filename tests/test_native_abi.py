@@ -159,6 +159,25 @@ def test_invalid_arguments_are_rejected_without_launch():
     assert L.ffa_kfmt_decode(ctypes.byref(k), None) == -2 and b"65535 workgroup spans" in L.ffa_last_error()
 
 
+@pytest.mark.parametrize("name", ["ffa_q2_quantize_g32_append_cast", "ffa_nvfp4_g16_append_cast", "ffa_nf4_g64_append_cast"])
+def test_cast_appends_reject_other_v_dtypes(name):
+    """V rows are fp16, bf16 or fp32 and the pool fp16 or bf16; anything else is refused before a launch (empty
+    dimensions are refused next, so the accepted pairs stop there)."""
+    from ffa_mi355x import _native as N
+
+    L = N.lib()
+    pools = 4 if "q2" in name else 3
+
+    def call(rows, pool):
+        return getattr(L, name)(64, 0, 0, 1, 1, 64, 64, 1, 1, *[64] * pools, 3, 64, rows, 64, pool, None)
+
+    for rows in (0, 1, 2):
+        for pool in (0, 1):
+            assert call(rows, pool) == -1 and b"bad dims" in L.ffa_last_error()
+    for rows, pool in ((0, 2), (1, 2), (2, 2), (3, 0), (4, 1), (3, 3), (-1, 0), (0, -1), (9, 9)):
+        assert call(rows, pool) == -1 and b"v dtypes" in L.ffa_last_error(), (rows, pool)
+
+
 def test_drop_in_signatures_match_reference():
     import attn_kernel.attn_kernel_v1210_fused_bsz_q2fp8 as K
 
