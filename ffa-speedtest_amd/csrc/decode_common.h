@@ -17,7 +17,7 @@ constexpr int kMinSpan = 2;                  // smallest span (chunks per workgr
 constexpr int kSmallSpanTokens = 8192;       // sequences up to this many tokens get slots for it
 // LDS row pitch (bytes) of a V tile staged row-major for the transposing reads (vt_operand_lds,
 // 8-byte aligned rows): whole tile (128 columns) 256 + 16; half a tile (64 columns) 128 + 8,
-// which keeps the q2 reference-layout decoder within two workgroups per CU (80.6 KB of LDS)
+// which keeps the q2 reference-layout decoder within two workgroups per CU (68.8 KB of LDS)
 constexpr int kVRow = 272;
 constexpr int kVRowHalf = 136;
 
@@ -117,7 +117,8 @@ __device__ __forceinline__ int div_bs(const DecodeParams &p, int x) {
 // layouts whose code lines hold several KV heads (the per-channel q2 rows, the 4-bit formats'
 // contiguous rows) keep the span fastest, so that the workgroups of one span's heads share each
 // line through one XCD's L2 (the unit first took the reference-layout config 2 from 16.1 to 17.9
-// us), and so does the other-format large-batch build (configs 3 and 4).  No division: the order
+// us; that placement needs a number of spans that is a multiple of 8, 64 there: with others the heads
+// of a span run on several XCDs, and only the last-level cache joins their lines), and so does the other-format large-batch build (configs 3 and 4).  No division: the order
 // is the grid's own (the position arithmetic of a rotated order cost config 2 0.2 us).
 struct GridPos {
   int cg, y, b;

@@ -437,8 +437,9 @@ __global__ __launch_bounds__(512) void kproj_rope_kernel(const void *h, const vo
 // staged through LDS.  (The kernel above keeps few tokens' W stream spread over the chip; with many it
 // reads h and W from the caches once per 32 channels and 16 tokens: 4096 tokens x 4096 -> 1024 take 249 us
 // there and 53 here, 0.65 PFLOP/s; the matrix cores need 23 at the rate a large product reaches.  What is
-// left: of a 64-wide step's 1320 cycles 512 are products, LDS moves 96 KB in another 515, partly under
-// them, and a wave has its SIMD to itself, so that every wait shows; 8 us are the first loads and the end.)
+// left: of a wave's 104 K cycles over 64 steps 33 K are products, LDS is busy for another 33 K with 96 KB a
+// step, partly under them (no bank conflicts), and a wave has its SIMD to itself, so that every wait shows;
+// 8 us are the first loads and the end.)
 //   * Four waves in 2 x 2 quarters; MFMA rows are channels and columns are tokens, so that a lane ends with
 //     four consecutive channels of one token: RoPE pairs need no exchange, stores are 16 bytes (fp32).
 //   * K in steps of 64: 16-byte pieces go to registers four steps ahead and to one of three LDS buffers two
