@@ -1,5 +1,5 @@
-"""The rules by which calls choose between kernels that give the same bytes (csrc/routes.h), on the CPU: at the sizes
-where each kernel was measured to be the faster one, the rule takes it."""
+"""The rules by which calls choose among kernels and builds that compute the same (csrc/routes.h), on the CPU: at the
+sizes where each was measured to be the faster one, the rule takes it."""
 import shutil
 import subprocess
 from pathlib import Path
